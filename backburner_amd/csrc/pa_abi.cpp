@@ -340,15 +340,24 @@ int attn_decode(Call & cx, const pa_hip_shape * s, const void * const * k_pages,
     return cx.merge(ma, (int) s->hd, st) ? 0 : -1;
 }
 
-// the matrix-core kernels: many rows per KV head at head dim 128 (verify, prefill: mma_kernel, row blocks of 32*NW
-// rows) and fp16-query calls at head dim 256 (mma256_kernel, row blocks of 64 rows), over chunks of 32-key tiles
+// the matrix-core kernels, over chunks of 32-key tiles: mma_kernel (row blocks of 32*NW rows) for every head-dim-128 call
+// that attn_decode does not take and for head dim 256 above 64 rows with fp16 operands; mma256_kernel (row blocks of 64
+// rows) for the other head-dim-256 calls
 int attn_mma(Call & cx, const pa_hip_shape * s, const void * const * k_pages, const void * const * v_pages,
              const uint32_t * nkeys, int n_pages, const float * Q, float * O, float * m, float * l, hipStream_t st) {
-    // head dim 128: 32 rows per wave, 8 waves above 128 rows (prefill), 4 otherwise (verify, short verify blocks, f16
-    // decode); head dim 256: 16 rows per wave, 4 waves (the reference's 48 rows per KV head fill three)
-    const bool h256 = s->hd == 256;
-    const uint32_t nw = h256 ? 4u : s->rows > 128 ? 8u : 4u, rpw = h256 ? 16u : 32u;
-    const uint32_t nrb = (s->rows + rpw * nw - 1) / (rpw * nw), qr = nrb * rpw * nw;
+    // mma_kernel: 32 rows per wave, 8 waves above 128 rows (prefill) and at head dim 256, 4 otherwise (verify, short verify
+    // blocks, f16 decode). mma256_kernel: 16 rows per wave, 4 waves (the reference's 48 rows per KV head fill three).
+    // Head dim 256 changes over where a second 64-row block would begin: each 16-row wave reads a whole tile from LDS for
+    // half the rows, and each 64-row block dequantizes it again. us per call, mma256_kernel against mma_kernel: 96 rows x
+    // 65,536 q8_0 keys 81 / 55, 192 rows x 32,768 q4_0 keys 68 / 55, 288 rows x 32,768 q8_0 keys (a second block of one
+    // wave) 99 / 89, 1,536 rows x 16,384 q4_0 keys 212 / 139; 48 rows stay (one 64-row block at two workgroups per CU, 49).
+    // The exact block dots (ggml's rounding over quantized K) need more registers there than 32 rows leave and stay too.
+    const bool h256 = s->hd == 256 && (s->rows <= 64 || (s->qmode == PA_QMODE_GGML && s->fmt != PA_FMT_F16));
+    const uint32_t nw = h256 ? 4u : s->rows > 128 || s->hd == 256 ? 8u : 4u, rpw = h256 ? 16u : 32u;
+    const uint32_t nrb = (s->rows + rpw * nw - 1) / (rpw * nw);
+    // rows per KV head in the slots: whole row blocks, at head dim 256 multiples of 64 under either kernel (only real rows
+    // are written)
+    const uint32_t qr = s->hd == 256 ? (s->rows + 63) / 64 * 64 : nrb * rpw * nw;
     // one row block with waves past the last row: those waves only stage (with several row blocks the full ones set
     // the time, and the staging-only branch would slow them)
     const bool skip = nrb == 1 && s->rows <= rpw * (nw - 1);
@@ -393,7 +402,7 @@ int attn_mma(Call & cx, const pa_hip_shape * s, const void * const * k_pages, co
         const uint32_t grid = (a.n_items + 7) / 8 * 8;
         hipEvent_t e0 = li == 0 ? cx.ev0 : nullptr, e1 = li + 1 == n_launch ? cx.ev1 : nullptr;
         ok = hip_ok(h256 ? launch_mma256((int) s->fmt, skip, a, grid, st, e0, e1)
-                         : launch_mma((int) s->fmt, (int) nw, skip, a, grid, st, e0, e1), "mma launch");
+                         : launch_mma((int) s->hd, (int) s->fmt, (int) nw, skip, a, grid, st, e0, e1), "mma launch");
         li++;
         slot0 += nch;
     });

@@ -1,5 +1,6 @@
 // pa_mma.hip - partial attention for many query rows per KV head (16-token verify, 512-token prefill chunks, and any
-// shape with more than 8 rows) over q8_0 / q4_0 / f16 K and V, head dim 128, fp16 matrix cores (gfx950).
+// shape with more than 8 rows) over q8_0 / q4_0 / f16 K and V, head dim 128 (and 256 above 64 rows with fp16 operands), on
+// the matrix cores (gfx950).
 //
 // One workgroup = one KV head x one block of 32*NW query rows x one chunk of consecutive 32-key tiles; NW waves, 32
 // rows each. Per tile the workgroup dequantizes V once into LDS as fp16 (d*q rounded once: the quants become fp16
@@ -9,8 +10,16 @@
 //   S^T (32 keys x 32 rows) = K . Q'^T      (8 MFMAs over the 128 dims; Q' stays in registers for the whole kernel),
 // so lane (h, n) holds row n's scores of keys 8j + 4h + i (j, i < 4) - which is exactly the B operand layout of
 //   O^T (128 dims x 32 rows) += V^T . P^T    (4 dim blocks x 2 MFMAs; V^T read from LDS by ds_read_b64_tr_b16),
-// so the probabilities never leave registers, and every value a lane holds belongs to its own row n: the running max
-// and sum need one exchange with lane n + 32 per tile and no LDS.
+// so the probabilities never leave registers, and every value a lane holds belongs to its own row n: each half row keeps its
+// own running max and sum, exchanged with lane n + 32 where the reference max moves and at the end only. At head dim 256 the
+// same with twice the MFMAs, K and V read from LDS a few operands ahead.
+//
+// What bounds it: a wave issues in order, and at two waves per SIMD its own chain of instructions per tile (about 190 vector
+// ones with the exact block dots, 90 without, at 4.5 cycles each, and 16 MFMAs of 32 cycles that they mostly wait for) is the
+// time, so what counts is the number of issued instructions on that chain and how evenly the two waves of a SIMD share the
+// staging. us per call, before and after the chain was shortened (scales of all blocks in one operand, dots converted by a
+// subtraction, page cursors of a few scalar additions, no lane exchange per tile, V staged by the older waves): 4,096 rows x 8
+// heads x 65,536 q8_0 keys 1,435 / 1,329, 128 rows x 8 heads x 98,304 q8_0 keys 104.8 / 101.0.
 //
 // Q' is the query as fp16: PA_QMODE_F16 takes fp16(q*scale) (the reference engines' Qs, phone-attn.h:595-599), and f16
 // K in PA_QMODE_GGML fp16(q), K's vec_dot type in ggml's CPU flash_attn_ext (the scale then multiplies the score).
@@ -29,25 +38,25 @@
 
 namespace pa_hip {
 
-constexpr int MM_HD = 128;
-constexpr int MM_KST = 2 * MM_HD + 16;            // K tile row stride (bytes): 16 consecutive keys' 16-byte reads hit
-                                                  // distinct banks
-constexpr int MM_VST = 2 * MM_HD + 64;            // V tile row stride: the 4 rows x 64 bytes of a half-wave's
-                                                  // transposing reads hit distinct banks
-constexpr int MM_KT = 32 * MM_KST, MM_VT = 32 * MM_VST;
-constexpr int MM_KST8 = MM_HD + 16;               // raw K tile row stride (EX): 16 consecutive keys' 16-byte
-                                                  // reads hit distinct banks
-constexpr int MM_KSC = 32 * 8;                    // exact-QK kernels: the tile's K block scales, [key][4 blocks] fp16
-constexpr int MM_STAGE = MM_KT + MM_VT + MM_KSC;
+// LDS geometry per head dim: K row stride 2 HD + 16 B (EX: the raw quants, HD + 16 B), so that 16 consecutive keys' 16-byte
+// reads hit distinct banks; V row stride 2 HD + 64 B, so that the 4 rows x 64 bytes of a half-wave's transposing reads do;
+// and for EX the tile's K block scales [key][HD / 32 blocks] fp16. A stage holds 19,200 B at head dim 128, 35,840 at 256.
+template <int HD> struct MmGeom {
+    static constexpr int NBLK = HD / 32;                      // quant blocks per head row
+    static constexpr int KST = 2 * HD + 16, KST8 = HD + 16, VST = 2 * HD + 64;
+    static constexpr int KT = 32 * KST, VT = 32 * VST, KSC = 32 * 2 * NBLK;
+    static constexpr int STAGE = KT + VT + KSC;
+};
 
 // The query rows as the fp16 B operand (lane (h2, n) holds row n, dims 16kk + 8h2 + t): f16(q * scale), or f16(q) for
 // f16 K in PA_QMODE_GGML (ggml's f16 vec_dot type)
-__device__ __forceinline__ void mm_prep_q(const AttnArgs & a, uint32_t h, uint32_t row, bool rlive, int h2, mm_h8 (&Qf)[8]) {
-    const float * qrow = a.q + ((size_t) h * a.rows + (rlive ? row : 0)) * MM_HD + 8 * h2;
+template <int HD>
+__device__ __forceinline__ void mm_prep_q(const AttnArgs & a, uint32_t h, uint32_t row, bool rlive, int h2, mm_h8 (&Qf)[HD / 16]) {
+    const float * qrow = a.q + ((size_t) h * a.rows + (rlive ? row : 0)) * HD + 8 * h2;
     const uint32_t qmask = rlive ? 0xffffffffu : 0u;
     const float qs = a.qmode == 0 ? 1.0f : a.scale;
     #pragma unroll
-    for (int kk = 0; kk < 8; kk++) {
+    for (int kk = 0; kk < HD / 16; kk++) {
         const pa_f4 x0 = __builtin_bit_cast(pa_f4, __builtin_bit_cast(pa_u4, *(const pa_f4 *) (qrow + 16 * kk)) & qmask);
         const pa_f4 x1 = __builtin_bit_cast(pa_f4, __builtin_bit_cast(pa_u4, *(const pa_f4 *) (qrow + 16 * kk + 4)) & qmask);
         mm_h8 f;
@@ -66,14 +75,14 @@ __device__ __forceinline__ void mm_prep_q(const AttnArgs & a, uint32_t h, uint32
 // For q4_0 K (unsigned nibbles u = q + 8 in the int8 MFMA) it also gives, per block, the (hi, lo) pair of
 // -8 * (sum of the row's block quants) * (hi + lo) in fp32 (dcb[b]): the offset the unsigned nibbles add to each block
 // dot, times the row's scale pair; a key's block scale times it is that block's correction of the score.
-template <int FMT>
-__device__ __forceinline__ void mm_prep_qi8(const AttnArgs & a, uint32_t h, uint32_t row, bool rlive, int h2, pa_u4 (&Qi)[4],
-                                            uint32_t (&dqb)[4], uint32_t (&dcb)[4]) {
-    const float * qrow = a.q + ((size_t) h * a.rows + (rlive ? row : 0)) * MM_HD + 16 * h2;
+template <int HD, int FMT>
+__device__ __forceinline__ void mm_prep_qi8(const AttnArgs & a, uint32_t h, uint32_t row, bool rlive, int h2, pa_u4 (&Qi)[HD / 32],
+                                            uint32_t (&dqb)[HD / 32], uint32_t (&dcb)[HD / 32]) {
+    const float * qrow = a.q + ((size_t) h * a.rows + (rlive ? row : 0)) * HD + 16 * h2;
     const uint32_t qmask = rlive ? 0xffffffffu : 0u;
     const float scale = a.scale;
     #pragma unroll
-    for (int b = 0; b < 4; b++) {
+    for (int b = 0; b < HD / 32; b++) {
         #pragma clang fp contract(off)
         pa_f4 x[4];
         #pragma unroll
@@ -113,16 +122,17 @@ __device__ __forceinline__ void mm_prep_qi8(const AttnArgs & a, uint32_t h, uint
 
 // Row n's result: the sum over both lanes, O rebased from the reference max to the exact one; the final (O, m, l)
 // for a single-chunk call, else split-K slot c
-__device__ __forceinline__ void mm_write_out(const AttnArgs & a, const mm_f16 (&O)[4], float mref, float mx, float lsum,
+template <int HD>
+__device__ __forceinline__ void mm_write_out(const AttnArgs & a, const mm_f16 (&O)[HD / 32], float mref, float mx, float lsum,
                                              uint32_t h, uint32_t row, bool rlive, int h2, uint32_t c) {
     const float lt = mm_sum32(lsum);
     const float f = mref == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mref - mx);
     if (!rlive) return;
     const bool direct = a.n_chunks == 1 && a.fused;
-    float * dst = direct ? a.O + ((size_t) h * a.rows + row) * MM_HD
-                         : a.po + (((size_t) h * a.qr + row) * a.slots + a.slot0 + c) * MM_HD;
+    float * dst = direct ? a.O + ((size_t) h * a.rows + row) * HD
+                         : a.po + (((size_t) h * a.qr + row) * a.slots + a.slot0 + c) * HD;
     #pragma unroll
-    for (int db = 0; db < 4; db++)
+    for (int db = 0; db < HD / 32; db++)
         #pragma unroll
         for (int j = 0; j < 4; j++) {
             const pa_f4 v = {O[db][4 * j] * f, O[db][4 * j + 1] * f, O[db][4 * j + 2] * f, O[db][4 * j + 3] * f};
@@ -142,8 +152,8 @@ __device__ __forceinline__ void mm_write_out(const AttnArgs & a, const mm_f16 (&
 // tile's fp16 block scales beside it (q8_0: the int8 quants as they are, half the LDS bytes of the fp16 tile; q4_0: the
 // nibbles of one block half as unsigned bytes u = q + 8), and Q as ggml's q8_0 int8 quants. Per 32-block b one
 // v_mfma_i32_32x32x32_i8 gives the integer dot itself (|dot| < 2^21), converted to fp32 exactly, and one fp16 MFMA the
-// scale product dk_b(key) * (hi + lo)(row): dk_b at k = 0 and 1 of A, the row's pair at k = 0 and 1 of B (an outer
-// product in otherwise zero operands). The scores are the fp32 sum over the blocks of dot_b * (scale product), started
+// scale product dk_b(key) * (hi + lo)(row) (an outer product: A holds every block's dk twice, block b's B
+// operand the row's pair at that block's two places and zeros elsewhere). The scores are the fp32 sum over the blocks of dot_b * (scale product), started
 // at -mref: ggml's per-block vec_dot arithmetic (vec_dot_q8_0_q8_0 / q4_0_q8_0), with the softmax scale and the base-2
 // conversion inside each block's factor instead of the dot of two fp16-rounded operands. For q4_0 the start value also
 // takes the offset of the unsigned nibbles, sum_b dk_b * (-8 * qsum_b) * (hi + lo)_b, from one more MFMA per tile.
@@ -153,14 +163,18 @@ __device__ __forceinline__ void mm_write_out(const AttnArgs & a, const mm_f16 (&
 // stores, and the barriers). For calls with one row block narrower than 32 * NW rows. Without SKIP there is no branch
 // there: one costs 13-20 % on full row blocks, as it separates the next tile's loads from the QK MFMAs, which the
 // compiler otherwise schedules in one basic block.
-template <int FMT, int NW, bool SKIP, bool EX>
+template <int HD, int FMT, int NW, bool SKIP, bool EX>
 __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) {   // 2 waves per SIMD
-    static_assert(!EX || FMT != 0, "the exact block dots take quantized K");
-    constexpr int PF = 2;                                            // tiles whose raw bytes are in flight
+    static_assert(!EX || (FMT != 0 && HD == 128), "the exact block dots take quantized K at head dim 128");
+    using G = MmGeom<HD>;
+    constexpr int NBLK = G::NBLK;
+    // tiles whose raw bytes are in flight in registers (head dim 256: one; O and Q take 192 of the 256 registers there, and
+    // a tile's matrix work is twice as long)
+    constexpr int PF = HD == 128 ? 2 : 1;
     constexpr int NT = 64 * NW;
-    constexpr int UPT = 512 / NT;                                    // staging units per thread (512 per tile)
-    static_assert(UPT * NT == 512, "NW must be 4 or 8");
-    __shared__ __attribute__((aligned(16))) char smem[2 * MM_STAGE];
+    constexpr int UPT = 128 * NBLK / NT;                             // staging units per thread (128 NBLK per tile)
+    static_assert(UPT * NT == 128 * NBLK, "NW must be 4 or 8");
+    __shared__ __attribute__((aligned(16))) char smem[2 * G::STAGE];
 
     // ---- which (chunk, KV head, row block): row blocks fastest, so the workgroups that share a chunk's K/V run side
     // by side on one XCD (= blockIdx % 8 in dispatch order, which takes a contiguous item range) and share its L2
@@ -179,49 +193,76 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     const bool rlive = row < a.rows;
     const bool wlive = !SKIP || rb * (32 * NW) + 32 * wave < a.rows;    // uniform: the wave has a live row
 
-    MmCursor cl, cc;                                                 // the next tile to load / to compute
-    cl.init(a); cc.init(a);
-
-    // ---- staging units of this thread: u = tid + NT*i -> tensor u >> 8 (= (wave + NW*i) >> 2, uniform), key
-    // (u >> 3) & 31, block (u >> 1) & 3, half u & 1; rows past the page's end reload its last row (masked later)
+    // ---- staging units of this thread: u = tid + NT*i -> tensor u / (64 NBLK) (= (wave + NW*i) / NBLK, uniform),
+    // key u / (2 NBLK) & 31, block (u >> 1) & (NBLK - 1), half u & 1; rows past the page's end reload its last row (masked later)
     using F = MmFmt<FMT>;
-    MmRaw<FMT> R0[UPT], R1[UPT];                                     // tile t's raw bytes in R(t % 2)
-    // buffer loads: the tile's first row of this head as the scalar base, its rows up to the page's end as the range.
-    // Past the chunk's last tile (live false) the same loads go out with an empty range (no memory access, zeros), so
-    // that every step issues the same batch and the wait before a tile's dequant covers its own batch only.
-    auto load_tile = [&](MmRaw<FMT> (&R)[UPT], uint32_t tau, bool live) {
-        if (live) cl.seek(a, tau);
-        const uint32_t j0 = live ? 32 * (tau - cl.tb) : 0u;
-        const uint32_t last = live ? cl.nk - 1 - j0 : 0u;
+    // the tensor of unit i. With one unit per thread waves 0-3 stage V and waves 4-7 K: V costs the dequantization, and the
+    // SIMDs' issue favours the older of its two waves (w and w + 4), so the older one takes it
+    auto unit_tensor = [&](int i) { return UPT == 1 ? 1 - wave / NBLK : (wave + NW * i) / NBLK; };
+    MmRaw<FMT> R0[UPT], R1[UPT];                                     // tile t's raw bytes in R(t % PF)
+    uint32_t vo[UPT], vq[UPT];                                       // a unit's scale and value bytes in its tile
+    #pragma unroll
+    for (int i = 0; i < UPT; i++) {
+        const uint32_t u = tid + NT * i, key = (u / (2 * NBLK)) & 31, blk = (u >> 1) & (NBLK - 1), half = u & 1;
+        vo[i] = key * a.rs + blk * F::BB;
+        vq[i] = vo[i] + (FMT == 1 ? 2 + 16 * half : FMT == 2 ? 2 : 32 * half);
+    }
+    // ---- page cursors (scalar): the loads' (bases of the next tile's rows of this head, keys left in the page) and the
+    // matrix work's (keys left). Tiles are taken in order, so a tile costs a few scalar additions and the page table, whose
+    // scalar loads would also wait for the LDS operations in flight, is read when a page ends only.
+    // The first page comes by shift for uniform pages (a.ptl < 32), else by a walk, one scalar load's latency per page.
+    uint32_t lpg = 0;
+    if (a.ptl < 32u) lpg = min(t0 >> a.ptl, a.n_pages - 1);
+    else while (t0 >= a.cstart[lpg + 1]) lpg++;
+    const uint32_t j00 = 32 * (t0 - a.cstart[lpg]);
+    uint32_t lleft = a.pstart[lpg + 1] - a.pstart[lpg] - j00;
+    const size_t hoff = (size_t) h * a.hb;
+    const uint8_t * lk = a.kp[lpg] + hoff + (size_t) j00 * a.rs, * lv = a.vp[lpg] + hoff + (size_t) j00 * a.rs;
+    uint32_t cpg = lpg;
+    uint32_t cleft = lleft;
+    const uint32_t rs32 = 32 * a.rs;
+    // buffer loads: the tile's first row of this head as the scalar base, its rows up to the page's end as the range (rows
+    // past it read zeros and are masked later). Past the chunk's last tile (live false) the same loads go out with an empty
+    // range (no memory access, zeros), so that every step issues the same batch and the wait before a tile's dequant
+    // covers its own batch only.
+    auto load_tile = [&](MmRaw<FMT> (&R)[UPT], bool live) {
+        if (live && lleft == 0) {
+            do { lpg++; lleft = a.pstart[lpg + 1] - a.pstart[lpg]; } while (lleft == 0);
+            lk = a.kp[lpg] + hoff;
+            lv = a.vp[lpg] + hoff;
+            __builtin_amdgcn_s_waitcnt(0xc07f);                      // lgkmcnt(0): no scalar load left outstanding
+        }
         // the range covers the tile's rows only (at most 32 of rs bytes, rs < 2^26 by the host's check), so a page of
         // any size keeps the 32-bit byte count exact
-        const uint32_t nrec = live ? min(last + 1, 32u) * a.rs : 0u;
+        const uint32_t nrec = live ? (lleft < 32 ? lleft * a.rs : rs32) : 0u;
         #pragma unroll
         for (int i = 0; i < UPT; i++) {
-            const int u = tid + NT * i;
-            const int tensor = (wave + NW * i) >> 2, key = (u >> 3) & 31, blk = (u >> 1) & 3, half = u & 1;
-            const uint8_t * base = (tensor ? cl.vb : cl.kb) + (size_t) h * a.hb + (size_t) j0 * a.rs;
-            const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *) base, (short) 0, (int) nrec, 0x00020000);
-            mm_load_unit_buf<FMT>(R[i], rsrc, min((uint32_t) key, last) * a.rs + blk * F::BB, half);
+            const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *) (unit_tensor(i) ? lv : lk), (short) 0, (int) nrec, 0x00020000);
+            R[i].q[0] = __builtin_bit_cast(pa_u4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, vq[i], 0, 0));
+            if constexpr (FMT == 0) R[i].q[1] = __builtin_bit_cast(pa_u4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, vq[i] + 16, 0, 0));
+            R[i].d = FMT == 0 ? 0u : __builtin_amdgcn_raw_buffer_load_b16(rsrc, vo[i], 0, 0);
         }
+        lk += rs32;
+        lv += rs32;
+        lleft -= min(lleft, 32u);
     };
     auto store_tile = [&](const MmRaw<FMT> (&R)[UPT], int stage) {
-        char * st = smem + stage * MM_STAGE;
+        char * st = smem + stage * G::STAGE;
         #pragma unroll
         for (int i = 0; i < UPT; i++) {
             const int u = tid + NT * i;
-            const int tensor = (wave + NW * i) >> 2, key = (u >> 3) & 31, blk = (u >> 1) & 3, half = u & 1;
+            const int tensor = unit_tensor(i), key = (u / (2 * NBLK)) & 31, blk = (u >> 1) & (NBLK - 1), half = u & 1;
             pa_u4 lo, hi;
             if (EX && tensor == 0) {                                 // K: the raw int8 quants (q4_0: this half's
                                                                      // nibbles as unsigned bytes), the block scale beside
-                if (half == 0) *(uint16_t *) (st + MM_KT + MM_VT + 8 * key + 2 * blk) = (uint16_t) R[i].d;
+                if (half == 0) *(uint16_t *) (st + G::KT + G::VT + 2 * NBLK * key + 2 * blk) = (uint16_t) R[i].d;
                 pa_u4 q = R[i].q[0];
                 if constexpr (FMT == 2) q = (q >> (4 * half)) & 0x0f0f0f0fu;
-                *(pa_u4 *) (st + key * MM_KST8 + 32 * blk + 16 * half) = q;
+                *(pa_u4 *) (st + key * G::KST8 + 32 * blk + 16 * half) = q;
                 continue;
             }
             mm_dequant<FMT>(R[i], half, lo, hi);
-            char * dst = tensor ? st + MM_KT + key * MM_VST : st + key * MM_KST;
+            char * dst = tensor ? st + G::KT + key * G::VST : st + key * G::KST;
             dst += 2 * (32 * blk + 16 * half);
             *(pa_u4 *) dst = lo;
             *(pa_u4 *) (dst + 16) = hi;
@@ -229,33 +270,48 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     };
 
     // ---- the first two tiles' loads, then the query rows (B operand: lane (h2, n) holds row n, dims 16kk + 8h2 + t)
-    load_tile(R0, t0, true);
+    load_tile(R0, true);
     __builtin_amdgcn_sched_barrier(0);
-    load_tile(R1, t0 + 1, ntiles > 1);
+    if constexpr (PF == 2) load_tile(R1, ntiles > 1);
     __builtin_amdgcn_sched_barrier(0);
-    mm_h8 Qf[8];                                                     // !EX: fp16 query operands
-    pa_u4 Qi[4];                                                     // EX: int8 query quants per block
-    uint32_t dqb[4] = {0u, 0u, 0u, 0u};                              // EX: the scale pairs
-    uint32_t dcb[4] = {0u, 0u, 0u, 0u};                              // EX, q4_0: the nibble-offset correction pairs
-    if constexpr (EX) mm_prep_qi8<FMT>(a, h, row, rlive, h2, Qi, dqb, dcb);
-    else mm_prep_q(a, h, row, rlive, h2, Qf);
-    // EX: the B operand of the scale products, the (hi, lo) pair of row n at k = 0, 1 (lanes h2 = 0), zero elsewhere
-    uint32_t dqw[4], dcw[4];
+    mm_h8 Qf[HD / 16];                                               // !EX: fp16 query operands
+    pa_u4 Qi[NBLK];                                                  // EX: int8 query quants per block
+    uint32_t dqb[NBLK], dcb[NBLK];                                   // EX: the scale pairs; q4_0: the nibble-offset pairs
     #pragma unroll
-    for (int b = 0; b < 4; b++) { dqw[b] = h2 == 0 ? dqb[b] : 0u; dcw[b] = h2 == 0 ? dcb[b] : 0u; }
-    // EX, q4_0: the correction MFMA's terms k = 8, 9 (lanes h2 = 1) are 1.0 x the (hi, lo) pair of -mref, so its
-    // result starts the scores at -mref; mref is kept at values the pair holds exactly
-    const uint32_t onew = h2 == 1 ? 0x3C003C00u : 0u;
+    for (int b = 0; b < NBLK; b++) dqb[b] = dcb[b] = 0u;
+    if constexpr (EX) mm_prep_qi8<HD, FMT>(a, h, row, rlive, h2, Qi, dqb, dcb);
+    else mm_prep_q<HD>(a, h, row, rlive, h2, Qf);
+    // EX: the B operands of the scale products. All four products share one A operand, key n's block scales at k = 2b and
+    // 2b + 1 (lanes h2 = b / 2, register b % 2), so block b's B operand holds row n's (hi, lo) pair there, zero elsewhere
+    // (one operand per block in otherwise zero registers took four permutes, four selects and eleven moves per tile more)
+    pa_u2 dqw[NBLK];
+    #pragma unroll
+    for (int b = 0; b < NBLK; b++) {
+        const uint32_t x = h2 == (b >> 1) ? dqb[b] : 0u;
+        dqw[b] = (b & 1) ? (pa_u2){0u, x} : (pa_u2){x, 0u};
+    }
+    // EX, q4_0: the correction MFMA's B operand has every block's pair at its place, and its terms k = 4, 5 of lanes
+    // h2 = 0 are 1.0 x the (hi, lo) pair of -mref, so its result starts the scores at -mref; mref is kept at values the
+    // pair holds exactly
+    const uint32_t onew = h2 == 0 ? 0x3C003C00u : 0u;
+    const pa_u2 dcw = h2 == 0 ? (pa_u2){dcb[0], dcb[1]} : (pa_u2){dcb[2], dcb[3]};
     uint32_t mcw = 0u;
+    // EX: the integer dots' start value, whose sum with a dot is the bits of the float 1.5 * 2^23 + dot (|dot| < 2^21): a
+    // subtraction then converts it exactly, at twice the rate of v_cvt_f32_i32 (1.0 against 1.8 ns per wave instruction
+    // and SIMD with two waves)
+    mm_i16 cvt0;
+    #pragma unroll
+    for (int v = 0; v < 16; v++) cvt0[v] = 0x4B400000;
+    if constexpr (EX) asm volatile("" : "+v"(cvt0));         // kept in registers, not rebuilt for every tile
 
     // ---- prologue: tile t0 -> stage 0, tile t0 + 2's loads in flight in R0 (t0 + 1's in R1)
     store_tile(R0, 0);
-    load_tile(R0, t0 + PF, ntiles > PF);
+    load_tile(R0, ntiles > PF);
     mm_lds_barrier();
 
-    mm_f16 O[4];
+    mm_f16 O[NBLK];
     #pragma unroll
-    for (int db = 0; db < 4; db++) O[db] = (mm_f16){};
+    for (int db = 0; db < NBLK; db++) O[db] = (mm_f16){};
     float mref = -INFINITY, mx = -INFINITY, lsum = 0.0f;
     const float sm = a.qmode == 0 && FMT == 0 ? a.scale * MM_LOG2E : MM_LOG2E;   // score -> base-2 logit (!EX)
     float mc = 0.0f;                                                 // EX: mref once it is finite (0 before), the shift
@@ -263,70 +319,75 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     const mm_h2 one2 = {(_Float16) 1.0f, (_Float16) 1.0f};
 
     const int q4 = lane >> 4, s4 = lane & 15;
+    // a tile's K operands (A operand of S^T, lane (h2, n): key n; !EX: dims 16kk + 8h2 .. +7; EX: the quants of dims 32b +
+    // 16h2 .. +15 and the scales of blocks 2 h2, 2 h2 + 1)
+    constexpr int KA = HD == 128 ? 8 : FMT == 0 ? 2 : 3;                           // !EX: K operands read ahead (of HD / 16)
+    mm_h8 kf[KA];
+    pa_u4 kq[4];
+    uint32_t dk2 = 0u;
+    auto kf_read = [&](const char * Kt, int kk) { kf[kk % KA] = *(const mm_h8 *) (Kt + n * G::KST + 32 * kk + 16 * h2); };
+    auto k_read = [&](int stage) {
+        const char * Kt = smem + stage * G::STAGE;
+        if constexpr (EX) {
+            dk2 = *(const uint32_t *) (Kt + G::KT + G::VT + 8 * n + 4 * h2);
+            #pragma unroll
+            for (int b = 0; b < 4; b++) kq[b] = *(const pa_u4 *) (Kt + n * G::KST8 + 32 * b + 16 * h2);
+        } else {
+            #pragma unroll
+            for (int kk = 0; kk < KA; kk++) kf_read(Kt, kk);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
     // one tile's matrix work on LDS stage `stage` (nvalid keys)
     auto compute = [&](int stage, int nvalid) {
-        const char * Kt = smem + stage * MM_STAGE;
-        const char * Vt = Kt + MM_KT;
+        const char * Kt = smem + stage * G::STAGE;
+        const char * Vt = Kt + G::KT;
 
-        // ---- LDS reads: K (A operand of S^T, lane (h2, n): key n, dims 16kk + 8h2 .. +7) first; V^T per dim block
-        // and 16-key half by two transposing reads (lane 16q + s reads key row 16mi + (8 for the second read) +
-        // 4(q >> 1) + s / 4, dims 32db + 16(q & 1) + 4(s % 4) .. +3), which complete under the softmax
-        __builtin_amdgcn_s_waitcnt(0xc07f);                          // lgkmcnt(0): the stores and any scalar load done,
-        mm_h8 kf[8];                                                 // so the MFMAs below wait for their own reads only
-        if constexpr (!EX) {
-            #pragma unroll
-            for (int kk = 0; kk < 8; kk++) kf[kk] = *(const mm_h8 *) (Kt + n * MM_KST + 32 * kk + 16 * h2);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        // ---- S^T = K Q'^T, each MFMA followed by the two transposing V reads of one (dim block, key half), so that at
-        // most 15 LDS reads are outstanding (the counter's range) and each MFMA waits for its own K read only
+        // V^T per (dim block db, 16-key half mi), idx = 2 db + mi, by two transposing reads (lane 16q + s reads key row 16mi +
+        // (8 for the second read) + 4(q >> 1) + s / 4, dims 32db + 16(q & 1) + 4(s % 4) .. +3). Head dim 128 holds all of
+        // them, read under the QK MFMAs and the softmax; head dim 256 reads VA ahead
+        constexpr int VA = HD == 128 ? 8 : FMT == 0 ? 2 : 3;
+        if constexpr (HD == 256) k_read(stage);
         mm_f16 S = (mm_f16){};
-        mm_h8 va[4][2];
-        auto v_read = [&](int kk) {
-            const int db = kk >> 1, mi = kk & 1;
-            const char * vb = Vt + (16 * mi + 4 * (q4 >> 1) + (s4 >> 2)) * MM_VST + 2 * (32 * db + 16 * (q4 & 1) + 4 * (s4 & 3));
+        mm_h8 va[VA];
+        auto v_read = [&](int idx) {
+            const int db = idx >> 1, mi = idx & 1;
+            const char * vb = Vt + (16 * mi + 4 * (q4 >> 1) + (s4 >> 2)) * G::VST + 2 * (32 * db + 16 * (q4 & 1) + 4 * (s4 & 3));
             const pa_h4 x0 = __builtin_bit_cast(pa_h4, __builtin_amdgcn_ds_read_tr16_b64_v4f16((MM_LDS mm_tr4 *) vb));
-            const pa_h4 x1 = __builtin_bit_cast(pa_h4, __builtin_amdgcn_ds_read_tr16_b64_v4f16((MM_LDS mm_tr4 *) (vb + 8 * MM_VST)));
-            va[db][mi] = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
+            const pa_h4 x1 = __builtin_bit_cast(pa_h4, __builtin_amdgcn_ds_read_tr16_b64_v4f16((MM_LDS mm_tr4 *) (vb + 8 * G::VST)));
+            va[idx % VA] = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
         };
         if constexpr (EX) {
             // per block: the integer dot on the int8 matrix cores (A: key n's quants, dims 32b + 16h2 .. +15, read raw
             // from the tile; B: the query quants), the scale product, and dot * product summed in fp32
-            const pa_u2 dk2 = *(const pa_u2 *) (Kt + MM_KT + MM_VT + 8 * n);   // key n's four fp16 block scales
-            const uint32_t hmask = h2 == 0 ? 0xffffffffu : 0u;
-            pa_u4 kq[4];
-            #pragma unroll
-            for (int b = 0; b < 4; b++) kq[b] = *(const pa_u4 *) (Kt + n * MM_KST8 + 32 * b + 16 * h2);
-            uint32_t dkw4[4];
-            #pragma unroll
-            for (int b = 0; b < 4; b++) dkw4[b] = pa_perm(0u, dk2[b >> 1], (b & 1) ? 0x03020302u : 0x01000100u) & hmask;
+            const pa_u2 dkw = {pa_perm(0u, dk2, 0x01000100u), pa_perm(0u, dk2, 0x03020302u)};
             if constexpr (FMT == 2) {
                 // q4_0: the scores start at -mref plus sum_b dk_b(key) * (-8 * qsum_b * dq_b)(row), one MFMA over the
-                // blocks' (hi, lo) pairs (k = 2b, 2b + 1) and -mref (k = 8, 9), so that the unsigned nibble dots need no
-                // per-score offset
-                S = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                    __builtin_bit_cast(mm_h8, (pa_u4){dkw4[0] | onew, dkw4[1], dkw4[2], dkw4[3]}),
-                    __builtin_bit_cast(mm_h8, (pa_u4){dcw[0] | mcw, dcw[1], dcw[2], dcw[3]}), (mm_f16){}, 0, 0, 0);
+                // blocks' (hi, lo) pairs and -mref, so that the unsigned nibble dots need no per-score offset
+                S = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(mm_h8, (pa_u4){dkw.x, dkw.y, onew, 0u}),
+                                                           __builtin_bit_cast(mm_h8, (pa_u4){dcw.x, dcw.y, mcw, 0u}),
+                                                           (mm_f16){}, 0, 0, 0);
             }
             #pragma unroll
             for (int b = 0; b < 4; b++) {
-                const mm_i16 T = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(mm_i4, kq[b]), __builtin_bit_cast(mm_i4, Qi[b]),
-                                                                     (mm_i16){}, 0, 0, 0);
-                const uint32_t dkw = dkw4[b];
-                const mm_f16 Pb = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(mm_h8, (pa_u4){dkw, 0u, 0u, 0u}),
-                                                                         __builtin_bit_cast(mm_h8, (pa_u4){dqw[b], 0u, 0u, 0u}),
-                                                                         (mm_f16){}, 0, 0, 0);
+                const mm_f16 T = __builtin_bit_cast(mm_f16, __builtin_amdgcn_mfma_i32_32x32x32_i8(
+                    __builtin_bit_cast(mm_i4, kq[b]), __builtin_bit_cast(mm_i4, Qi[b]), cvt0, 0, 0, 0));
+                const mm_f16 Pb = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(pa_h4, dkw), __builtin_bit_cast(pa_h4, dqw[b]),
+                                                                       (mm_f16){}, 0, 0, 0);
                 #pragma unroll
-                for (int v = 0; v < 16; v++) S[v] = fmaf(Pb[v], (float) T[v], b == 0 && FMT == 1 ? -mc : S[v]);
+                for (int v = 0; v < 16; v++) S[v] = fmaf(Pb[v], T[v] - 12582912.0f, b == 0 && FMT == 1 ? -mc : S[v]);
                 __builtin_amdgcn_sched_barrier(0);
             }
             #pragma unroll
-            for (int kk = 0; kk < 8; kk++) v_read(kk);               // V^T after the block dots, under the softmax
+            for (int i = 0; i < VA; i++) v_read(i);                  // V^T after the block dots, under the softmax
         } else {
+            // S^T = K Q'^T; at head dim 128 each MFMA is followed by the two transposing V reads of one (dim block, key half),
+            // so that at most 15 LDS reads are outstanding (the counter's range) and each MFMA waits for its own K read only
             #pragma unroll
-            for (int kk = 0; kk < 8; kk++) {
-                S = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[kk], Qf[kk], S, 0, 0, 0);
-                v_read(kk);
+            for (int kk = 0; kk < HD / 16; kk++) {
+                S = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[kk % KA], Qf[kk], S, 0, 0, 0);
+                if (kk + KA < HD / 16) kf_read(Kt, kk + KA);
+                if (kk >= HD / 16 - VA) v_read(kk - (HD / 16 - VA));
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -335,22 +396,25 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
             for (int v = 0; v < 16; v++)
                 if (8 * (v / 4) + 4 * h2 + (v % 4) >= nvalid) S[v] = -INFINITY;
         }
-        float tm = S[0];
-        #pragma unroll
-        for (int v = 1; v < 16; v++) tm = fmaxf(tm, S[v]);
-        tm = EX ? mm_max32(tm) + mc : mm_max32(tm) * sm;             // row n's tile max, base 2
+        float tm = fmaxf(fmaxf(S[0], S[1]), S[2]);                   // this lane's half of row n's tile max
+        {
+            const float t1 = fmaxf(fmaxf(S[3], S[4]), S[5]), t2 = fmaxf(fmaxf(S[6], S[7]), S[8]), t3 = fmaxf(fmaxf(S[9], S[10]), S[11]),
+                        t4 = fmaxf(fmaxf(S[12], S[13]), S[14]);
+            tm = fmaxf(fmaxf(fmaxf(tm, t1), t2), fmaxf(fmaxf(t3, t4), S[15]));
+        }
+        tm = EX ? tm + mc : tm * sm;                                 // base 2
         if (__builtin_amdgcn_ballot_w64(tm > mref + MM_PMAX)) {
             // rare: move the reference max of every row that needs it (uniform branch)
-            float mn = fmaxf(mref, tm);
+            float mn = fmaxf(mref, mm_max32(tm));                    // the row's other half: lane ^ 32
             if constexpr (EX && FMT == 2) {                          // a value the (hi, lo) pair of -mn holds exactly
                 const _Float16 mh = (_Float16) mn, ml = (_Float16) (mn - (float) mh);
                 mn = (float) mh + (float) ml;
                 const _Float16 nh = -mh, nl = -ml;
-                mcw = h2 == 1 ? (uint32_t) __builtin_bit_cast(uint16_t, nh) | ((uint32_t) __builtin_bit_cast(uint16_t, nl) << 16) : 0u;
+                mcw = h2 == 0 ? (uint32_t) __builtin_bit_cast(uint16_t, nh) | ((uint32_t) __builtin_bit_cast(uint16_t, nl) << 16) : 0u;
             }
             const float alpha = mref == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mref - mn);
             #pragma unroll
-            for (int db = 0; db < 4; db++) O[db] *= alpha;
+            for (int db = 0; db < NBLK; db++) O[db] *= alpha;
             lsum *= alpha;
             mref = mn;
             if constexpr (EX) {                                      // rebase this tile's scores and the start value
@@ -373,61 +437,91 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
 
         // ---- O^T += V^T P^T
         #pragma unroll
-        for (int db = 0; db < 4; db++)
-            #pragma unroll
-            for (int mi = 0; mi < 2; mi++) O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[db][mi], P[mi], O[db], 0, 0, 0);
+        for (int i = 0; i < 2 * NBLK; i++) {
+            O[i >> 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[i % VA], P[i & 1], O[i >> 1], 0, 0, 0);
+            if (i + VA < 2 * NBLK) v_read(i + VA);
+        }
     };
     // one tile step; Rn holds tile t + 1's raw bytes
     auto step = [&](uint32_t t, MmRaw<FMT> (&Rn)[UPT]) {
         const int stage = t & 1;
-        const uint32_t tau = t0 + t;
-        cc.seek(a, tau);                                             // before any LDS operation of this step
-        const int nvalid = (int) min(32u, cc.nk - 32 * (tau - cc.tb));
+        if (cleft == 0) {                                            // before any LDS operation of this step
+            do { cpg++; cleft = a.pstart[cpg + 1] - a.pstart[cpg]; } while (cleft == 0);
+            __builtin_amdgcn_s_waitcnt(0xc07f);
+        }
+        const int nvalid = (int) min(32u, cleft);
+        cleft -= nvalid;
         // the next tile's bytes -> the other stage (last read before the previous barrier; past the chunk's end the
         // stage is written and never read), then tile t + 1 + PF's loads into the registers just freed
-        const bool nlive = t + 1 + PF < ntiles;
-        if (nlive) cl.seek(a, tau + 1 + PF);
+        if (HD == 128 && wlive) k_read(stage);
         store_tile(Rn, stage ^ 1);
-        load_tile(Rn, tau + 1 + PF, nlive);
+        load_tile(Rn, t + 1 + PF < ntiles);
         if (wlive) compute(stage, nvalid);
         mm_lds_barrier();                                            // this stage is free; the next one is written
     };
-    uint32_t t = 0;                                                  // tile t + 1 is in R((t + 1) % 2)
-    for (; t + 2 <= ntiles; t += 2) {
-        step(t, R1);
-        step(t + 1, R0);
+    uint32_t t = 0;                                                  // tile t + 1 is in R((t + 1) % PF)
+    if constexpr (PF == 2) {
+        for (; t + 2 <= ntiles; t += 2) {
+            step(t, R1);
+            step(t + 1, R0);
+        }
+        if (t < ntiles) step(t, R1);
+    } else {
+        for (; t < ntiles; t++) step(t, R0);
     }
-    if (t < ntiles) step(t, R1);
 
-    mm_write_out(a, O, mref, mx, lsum, h, row, rlive, h2, c);
+    mx = mm_max32(mx);                                               // the exact row max, tracked per half row
+    mm_write_out<HD>(a, O, mref, mx, lsum, h, row, rlive, h2, c);
 }
 
 // The ggml query rounding over quantized K takes the exact block dots at every size (4-wave verify blocks and 8-wave
 // prefill chunks); the reference engines' rounding (PA_QMODE_F16) and f16 K take the fp16-operand QK, the Metal
 // engine's own arithmetic (K dequantized to half in threadgroup memory, pa-metal.mm:379-487)
-template <int FMT, bool EX>
+template <int HD, int FMT, bool EX>
 static hipError_t launch_mma_fmt(int nw, bool skip, const AttnArgs & a, uint32_t grid, hipStream_t st, hipEvent_t ev0,
                                  hipEvent_t ev1) {
     switch (nw) {
         case 4:
-            if (skip) hipExtLaunchKernelGGL((mma_kernel<FMT, 4, true, EX>), dim3(grid), dim3(256), 0, st, ev0, ev1, 0, a);
-            else hipExtLaunchKernelGGL((mma_kernel<FMT, 4, false, EX>), dim3(grid), dim3(256), 0, st, ev0, ev1, 0, a);
+            if (skip) hipExtLaunchKernelGGL((mma_kernel<HD, FMT, 4, true, EX>), dim3(grid), dim3(256), 0, st, ev0, ev1, 0, a);
+            else hipExtLaunchKernelGGL((mma_kernel<HD, FMT, 4, false, EX>), dim3(grid), dim3(256), 0, st, ev0, ev1, 0, a);
             break;
         case 8:
-            if (skip) hipExtLaunchKernelGGL((mma_kernel<FMT, 8, true, EX>), dim3(grid), dim3(512), 0, st, ev0, ev1, 0, a);
-            else hipExtLaunchKernelGGL((mma_kernel<FMT, 8, false, EX>), dim3(grid), dim3(512), 0, st, ev0, ev1, 0, a);
+            if (skip) hipExtLaunchKernelGGL((mma_kernel<HD, FMT, 8, true, EX>), dim3(grid), dim3(512), 0, st, ev0, ev1, 0, a);
+            else hipExtLaunchKernelGGL((mma_kernel<HD, FMT, 8, false, EX>), dim3(grid), dim3(512), 0, st, ev0, ev1, 0, a);
             break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
 
-hipError_t launch_mma(int fmt, int nw, bool skip, const AttnArgs & a, uint32_t grid, hipStream_t st, hipEvent_t ev0,
-                      hipEvent_t ev1) {
+static hipError_t launch_mma_128(int fmt, int nw, bool skip, const AttnArgs & a, uint32_t grid, hipStream_t st, hipEvent_t ev0,
+                                 hipEvent_t ev1) {
     const bool ex = a.qmode == 0;                                    // PA_QMODE_GGML over quantized K: exact block dots
-    if (fmt == 0) return launch_mma_fmt<0, false>(nw, skip, a, grid, st, ev0, ev1);
-    if (fmt == 1) return ex ? launch_mma_fmt<1, true>(nw, skip, a, grid, st, ev0, ev1) : launch_mma_fmt<1, false>(nw, skip, a, grid, st, ev0, ev1);
-    if (fmt == 2) return ex ? launch_mma_fmt<2, true>(nw, skip, a, grid, st, ev0, ev1) : launch_mma_fmt<2, false>(nw, skip, a, grid, st, ev0, ev1);
+    if (fmt == 0) return launch_mma_fmt<128, 0, false>(nw, skip, a, grid, st, ev0, ev1);
+    if (fmt == 1) return ex ? launch_mma_fmt<128, 1, true>(nw, skip, a, grid, st, ev0, ev1) : launch_mma_fmt<128, 1, false>(nw, skip, a, grid, st, ev0, ev1);
+    if (fmt == 2) return ex ? launch_mma_fmt<128, 2, true>(nw, skip, a, grid, st, ev0, ev1) : launch_mma_fmt<128, 2, false>(nw, skip, a, grid, st, ev0, ev1);
+    return hipErrorInvalidValue;
+}
+
+template <int FMT>
+static hipError_t launch_mma_256_fmt(bool skip, const AttnArgs & a, uint32_t grid, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
+    if (skip) hipExtLaunchKernelGGL((mma_kernel<256, FMT, 8, true, false>), dim3(grid), dim3(512), 0, st, ev0, ev1, 0, a);
+    else hipExtLaunchKernelGGL((mma_kernel<256, FMT, 8, false, false>), dim3(grid), dim3(512), 0, st, ev0, ev1, 0, a);
+    return hipGetLastError();
+}
+
+static hipError_t launch_mma_256(int fmt, bool skip, const AttnArgs & a, uint32_t grid, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
+    if (fmt == 0) return launch_mma_256_fmt<0>(skip, a, grid, st, ev0, ev1);
+    if (a.qmode == 0) return hipErrorInvalidValue;                   // exact block dots at head dim 256: mma256_kernel
+    if (fmt == 1) return launch_mma_256_fmt<1>(skip, a, grid, st, ev0, ev1);
+    if (fmt == 2) return launch_mma_256_fmt<2>(skip, a, grid, st, ev0, ev1);
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_mma(int hd, int fmt, int nw, bool skip, const AttnArgs & a, uint32_t grid, hipStream_t st, hipEvent_t ev0,
+                      hipEvent_t ev1) {
+    if (hd == 128) return launch_mma_128(fmt, nw, skip, a, grid, st, ev0, ev1);
+    if (hd == 256 && nw == 8) return launch_mma_256(fmt, skip, a, grid, st, ev0, ev1);
     return hipErrorInvalidValue;
 }
 

@@ -82,6 +82,21 @@ def test_mma256_row_blocks(ws, fmt, rows):
     run_and_check(ws, fmt, 2, rows, 256, 1500, seed=700 + rows + fmt, qmode=bb.QMODE_F16, page_keys=512)
 
 
+@pytest.mark.parametrize("fmt", [bb.FMT_Q8_0, bb.FMT_Q4_0, bb.FMT_F16])
+@pytest.mark.parametrize("rows", [65, 224, 225, 257])
+@pytest.mark.parametrize("workgroups", [0, 1, 400])
+def test_head256_wide_rows(ws, fmt, rows, workgroups):
+    """Head dim 256 above 64 rows with fp16 operands (32-row waves, 256-row blocks): the first row past the 64-row blocks,
+    the last row count with idle waves, the first without, a second row block of one row; over pages that end inside a
+    tile, hold less than one or nothing, in the default chunks, in one chunk per row block (every page change inside the
+    workgroup) and in chunks of one tile."""
+    ws.set_split(mma_workgroups=workgroups)
+    try:
+        run_and_check(ws, fmt, 2, rows, 256, 1037, seed=1700 + rows + fmt, qmode=bb.QMODE_F16, page_keys=[500, 7, 0, 64, 466])
+    finally:
+        ws.set_split()
+
+
 @pytest.mark.parametrize("fmt", [bb.FMT_Q8_0, bb.FMT_F16])
 def test_mma256_split_invariance(ws, fmt):
     """The head-dim-256 kernel at the reference's 48 rows x 4 KV heads over chunks of 1, 2, 3, 5 and 40 tiles and one
