@@ -349,8 +349,8 @@ int attn_mma(Call & cx, const pa_hip_shape * s, const void * const * k_pages, co
     // blocks, f16 decode). mma256_kernel: 16 rows per wave, 4 waves (the reference's 48 rows per KV head fill three).
     // Head dim 256 changes over where a second 64-row block would begin: each 16-row wave reads a whole tile from LDS for
     // half the rows, and each 64-row block dequantizes it again. us per call, mma256_kernel against mma_kernel: 96 rows x
-    // 65,536 q8_0 keys 81 / 55, 192 rows x 32,768 q4_0 keys 68 / 55, 288 rows x 32,768 q8_0 keys (a second block of one
-    // wave) 99 / 89, 1,536 rows x 16,384 q4_0 keys 212 / 139; 48 rows stay (one 64-row block at two workgroups per CU, 49).
+    // 65,536 q8_0 keys 81 / 56, 192 rows x 32,768 q4_0 keys 68 / 55, 288 rows x 32,768 q8_0 keys (a second block of one
+    // wave) 99 / 89, 1,536 rows x 16,384 q4_0 keys 211 / 136; 48 rows stay (one 64-row block at two workgroups per CU, 49).
     // The exact block dots (ggml's rounding over quantized K) need more registers there than 32 rows leave and stay too.
     const bool h256 = s->hd == 256 && (s->rows <= 64 || (s->qmode == PA_QMODE_GGML && s->fmt != PA_FMT_F16));
     const uint32_t nw = h256 ? 4u : s->rows > 128 || s->hd == 256 ? 8u : 4u, rpw = h256 ? 16u : 32u;

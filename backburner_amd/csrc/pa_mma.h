@@ -117,6 +117,14 @@ __device__ __forceinline__ float mm_sum32(float v) {    // sum over lanes l and 
     return __builtin_bit_cast(float, (unsigned) t[0]) + __builtin_bit_cast(float, (unsigned) t[1]);
 }
 
+// A wave-uniform value kept in scalar registers. The compiler holds the results of uniform divisions in vector registers, and
+// what is computed from them after that: buffer descriptors then cost a readfirstlane per word and load.
+__device__ __forceinline__ uint32_t mm_uni(uint32_t v) { return (uint32_t) __builtin_amdgcn_readfirstlane((int) v); }
+__device__ __forceinline__ const uint8_t * mm_uni(const uint8_t * p) {
+    const uint64_t v = (uint64_t) p;
+    return (const uint8_t *) (((uint64_t) mm_uni((uint32_t) (v >> 32)) << 32) | mm_uni((uint32_t) v));
+}
+
 // Page cursor (scalar): the page holding a tile, its tile range and key count. A cursor moves only when a tile leaves
 // its page, so the common case reads no kernel argument memory (whose scalar loads would also wait for the LDS
 // operations in flight).

@@ -19,7 +19,7 @@
 // time, so what counts is the number of issued instructions on that chain and how evenly the two waves of a SIMD share the
 // staging. us per call, before and after the chain was shortened (scales of all blocks in one operand, dots converted by a
 // subtraction, page cursors of a few scalar additions, no lane exchange per tile, V staged by the older waves): 4,096 rows x 8
-// heads x 65,536 q8_0 keys 1,435 / 1,329, 128 rows x 8 heads x 98,304 q8_0 keys 104.8 / 101.0.
+// heads x 65,536 q8_0 keys 1,388 / 1,266, 128 rows x 8 heads x 98,304 q8_0 keys 101.3 / 95.1.
 //
 // Q' is the query as fp16: PA_QMODE_F16 takes fp16(q*scale) (the reference engines' Qs, phone-attn.h:595-599), and f16
 // K in PA_QMODE_GGML fp16(q), K's vec_dot type in ggml's CPU flash_attn_ext (the scale then multiplies the score).
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     const uint32_t t8 = (a.n_items + 7) / 8;
     const uint32_t w = xcd * t8 + local;
     if (local >= t8 || w >= a.n_items) return;
-    const uint32_t rb = w % a.nrb, h = (w / a.nrb) % a.nkv, c = w / (a.nrb * a.nkv);
+    const uint32_t rb = mm_uni(w % a.nrb), h = mm_uni((w / a.nrb) % a.nkv), c = mm_uni(w / (a.nrb * a.nkv));
     const uint32_t T = a.cstart[a.n_pages];                          // 32-key tiles of the call
     const uint32_t t0 = c * a.chunk, ntiles = min(t0 + a.chunk, T) - t0;   // this chunk's tiles [t0, t0 + ntiles)
 
@@ -214,27 +214,31 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     uint32_t lpg = 0;
     if (a.ptl < 32u) lpg = min(t0 >> a.ptl, a.n_pages - 1);
     else while (t0 >= a.cstart[lpg + 1]) lpg++;
+    lpg = mm_uni(lpg);
     const uint32_t j00 = 32 * (t0 - a.cstart[lpg]);
-    uint32_t lleft = a.pstart[lpg + 1] - a.pstart[lpg] - j00;
+    // tiles left in the page and the keys of its last one (no subtraction that stops at zero: that is a vector instruction
+    // here, and the descriptors built on its result would take a loop over the lanes per load)
+    uint32_t lkeys = mm_uni(a.pstart[lpg + 1] - a.pstart[lpg]), ltl = (lkeys - 1) / 32 + 1 - j00 / 32, llast = (lkeys - 1) % 32 + 1;
     const size_t hoff = (size_t) h * a.hb;
-    const uint8_t * lk = a.kp[lpg] + hoff + (size_t) j00 * a.rs, * lv = a.vp[lpg] + hoff + (size_t) j00 * a.rs;
-    uint32_t cpg = lpg;
-    uint32_t cleft = lleft;
+    const uint8_t * lk = mm_uni(a.kp[lpg] + hoff + (size_t) j00 * a.rs), * lv = mm_uni(a.vp[lpg] + hoff + (size_t) j00 * a.rs);
+    uint32_t cpg = lpg, ctl = ltl, clast = llast;
     const uint32_t rs32 = 32 * a.rs;
     // buffer loads: the tile's first row of this head as the scalar base, its rows up to the page's end as the range (rows
     // past it read zeros and are masked later). Past the chunk's last tile (live false) the same loads go out with an empty
     // range (no memory access, zeros), so that every step issues the same batch and the wait before a tile's dequant
     // covers its own batch only.
     auto load_tile = [&](MmRaw<FMT> (&R)[UPT], bool live) {
-        if (live && lleft == 0) {
-            do { lpg++; lleft = a.pstart[lpg + 1] - a.pstart[lpg]; } while (lleft == 0);
-            lk = a.kp[lpg] + hoff;
-            lv = a.vp[lpg] + hoff;
+        if (live && ltl == 0) {
+            do { lpg++; lkeys = a.pstart[lpg + 1] - a.pstart[lpg]; } while (lkeys == 0);
+            ltl = (lkeys - 1) / 32 + 1;
+            llast = (lkeys - 1) % 32 + 1;
+            lk = mm_uni(a.kp[lpg] + hoff);
+            lv = mm_uni(a.vp[lpg] + hoff);
             __builtin_amdgcn_s_waitcnt(0xc07f);                      // lgkmcnt(0): no scalar load left outstanding
         }
         // the range covers the tile's rows only (at most 32 of rs bytes, rs < 2^26 by the host's check), so a page of
         // any size keeps the 32-bit byte count exact
-        const uint32_t nrec = live ? (lleft < 32 ? lleft * a.rs : rs32) : 0u;
+        const uint32_t nrec = (live ? (ltl == 1 ? llast : 32u) : 0u) * a.rs;
         #pragma unroll
         for (int i = 0; i < UPT; i++) {
             const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *) (unit_tensor(i) ? lv : lk), (short) 0, (int) nrec, 0x00020000);
@@ -244,7 +248,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
         }
         lk += rs32;
         lv += rs32;
-        lleft -= min(lleft, 32u);
+        ltl -= 1;
     };
     auto store_tile = [&](const MmRaw<FMT> (&R)[UPT], int stage) {
         char * st = smem + stage * G::STAGE;
@@ -321,7 +325,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     const int q4 = lane >> 4, s4 = lane & 15;
     // a tile's K operands (A operand of S^T, lane (h2, n): key n; !EX: dims 16kk + 8h2 .. +7; EX: the quants of dims 32b +
     // 16h2 .. +15 and the scales of blocks 2 h2, 2 h2 + 1)
-    constexpr int KA = HD == 128 ? 8 : FMT == 0 ? 2 : 3;                           // !EX: K operands read ahead (of HD / 16)
+    constexpr int KA = HD == 128 ? 8 : FMT == 0 ? 2 : 3;              // !EX: K operands read ahead (of HD / 16)
+    constexpr bool KEARLY = HD == 128 && !SKIP;                      // read before the staging (the registers allow it)
     mm_h8 kf[KA];
     pa_u4 kq[4];
     uint32_t dk2 = 0u;
@@ -346,8 +351,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
         // V^T per (dim block db, 16-key half mi), idx = 2 db + mi, by two transposing reads (lane 16q + s reads key row 16mi +
         // (8 for the second read) + 4(q >> 1) + s / 4, dims 32db + 16(q & 1) + 4(s % 4) .. +3). Head dim 128 holds all of
         // them, read under the QK MFMAs and the softmax; head dim 256 reads VA ahead
-        constexpr int VA = HD == 128 ? 8 : FMT == 0 ? 2 : 3;
-        if constexpr (HD == 256) k_read(stage);
+        constexpr int VA = HD == 128 ? 8 : 2;
+        if constexpr (!KEARLY) k_read(stage);
         mm_f16 S = (mm_f16){};
         mm_h8 va[VA];
         auto v_read = [&](int idx) {
@@ -445,15 +450,18 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     // one tile step; Rn holds tile t + 1's raw bytes
     auto step = [&](uint32_t t, MmRaw<FMT> (&Rn)[UPT]) {
         const int stage = t & 1;
-        if (cleft == 0) {                                            // before any LDS operation of this step
-            do { cpg++; cleft = a.pstart[cpg + 1] - a.pstart[cpg]; } while (cleft == 0);
+        if (ctl == 0) {                                              // before any LDS operation of this step
+            uint32_t keys;
+            do { cpg++; keys = a.pstart[cpg + 1] - a.pstart[cpg]; } while (keys == 0);
+            ctl = (keys - 1) / 32 + 1;
+            clast = (keys - 1) % 32 + 1;
             __builtin_amdgcn_s_waitcnt(0xc07f);
         }
-        const int nvalid = (int) min(32u, cleft);
-        cleft -= nvalid;
+        const int nvalid = (int) (ctl == 1 ? clast : 32u);
+        ctl -= 1;
         // the next tile's bytes -> the other stage (last read before the previous barrier; past the chunk's end the
         // stage is written and never read), then tile t + 1 + PF's loads into the registers just freed
-        if (HD == 128 && wlive) k_read(stage);
+        if (KEARLY) k_read(stage);
         store_tile(Rn, stage ^ 1);
         load_tile(Rn, t + 1 + PF < ntiles);
         if (wlive) compute(stage, nvalid);
