@@ -401,8 +401,13 @@ int attn_mma(Call & cx, const pa_hip_shape * s, const void * const * k_pages, co
         a.q = Q; a.po = cx.po; a.pml = cx.pml; a.O = O; a.m = m; a.l = l;
         const uint32_t grid = (a.n_items + 7) / 8 * 8;
         hipEvent_t e0 = li == 0 ? cx.ev0 : nullptr, e1 = li + 1 == n_launch ? cx.ev1 : nullptr;
+        // two tile streams per workgroup (mma_kernel, NS) where half its waves have no rows and the chunk is long enough to
+        // pay for the fold: with 33-64 rows from about 10 tiles (us with one / two: 17 tiles 36.8 / 34.0, 6 tiles 25.1 /
+        // 25.9), up to 32 rows, where a quarter of the waves still idles, from about 32 (48 tiles 58.7 / 56.2, 17 tiles 30.5
+        // / 31.5)
+        const int streams = s->hd == 128 && s->rows <= 64 && tpc >= (s->rows > 32 ? 10u : 32u) ? 2 : 1;
         ok = hip_ok(h256 ? launch_mma256((int) s->fmt, skip, a, grid, st, e0, e1)
-                         : launch_mma((int) s->hd, (int) s->fmt, (int) nw, skip, a, grid, st, e0, e1), "mma launch");
+                         : launch_mma((int) s->hd, (int) s->fmt, (int) nw, skip, streams, a, grid, st, e0, e1), "mma launch");
         li++;
         slot0 += nch;
     });

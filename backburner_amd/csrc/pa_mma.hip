@@ -163,18 +163,25 @@ __device__ __forceinline__ void mm_write_out(const AttnArgs & a, const mm_f16 (&
 // stores, and the barriers). For calls with one row block narrower than 32 * NW rows. Without SKIP there is no branch
 // there: one costs 13-20 % on full row blocks, as it separates the next tile's loads from the QK MFMAs, which the
 // compiler otherwise schedules in one basic block.
-template <int HD, int FMT, int NW, bool SKIP, bool EX>
+// NS = 2 (SKIP, 4 waves, at most 64 rows, one row block): waves 0-1 and 2-3 are two streams that hold the same rows, a step
+// stages two tiles and stream x computes the tile 2t + x, where with one stream half the waves of the workgroup (and, as wave i
+// of every workgroup runs on SIMD i, half the SIMDs) only stage. The streams fold through LDS at the end, so the slots stay one
+// per workgroup. us per call with one stream and with two: 64 rows x 8 heads x 98,304 q4_0 keys 78.0 / 65.2, 40 rows x 33,333
+// q4_0 keys 36.8 / 34.0, 48 rows x 65,536 q4_0 keys (fp16 operands) 45.6 / 43.6.
+template <int HD, int FMT, int NW, bool SKIP, bool EX, int NS = 1>
 __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) {   // 2 waves per SIMD
     static_assert(!EX || (FMT != 0 && HD == 128), "the exact block dots take quantized K at head dim 128");
     using G = MmGeom<HD>;
     constexpr int NBLK = G::NBLK;
     // tiles whose raw bytes are in flight in registers (head dim 256: one; O and Q take 192 of the 256 registers there, and
     // a tile's matrix work is twice as long)
-    constexpr int PF = HD == 128 ? 2 : 1;
+    constexpr int PF = HD == 128 && NS == 1 ? 2 : 1;
     constexpr int NT = 64 * NW;
-    constexpr int UPT = 128 * NBLK / NT;                             // staging units per thread (128 NBLK per tile)
+    constexpr int UPT = 128 * NBLK / NT;                             // staging units per thread and tile (128 NBLK per tile)
+    constexpr int RW = NW / NS;                                      // row waves per stream
+    static_assert(NS == 1 || (SKIP && HD == 128), "several streams come with one partly filled row block");
     static_assert(UPT * NT == 128 * NBLK, "NW must be 4 or 8");
-    __shared__ __attribute__((aligned(16))) char smem[2 * G::STAGE];
+    __shared__ __attribute__((aligned(16))) char smem[2 * NS * G::STAGE];
 
     // ---- which (chunk, KV head, row block): row blocks fastest, so the workgroups that share a chunk's K/V run side
     // by side on one XCD (= blockIdx % 8 in dispatch order, which takes a contiguous item range) and share its L2
@@ -189,9 +196,10 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     const int tid = threadIdx.x, lane = tid % 64;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int n = lane & 31, h2 = lane >> 5;
-    const uint32_t row = rb * (32 * NW) + 32 * wave + n;             // this lane's query row (within the KV head)
+    const int rw = wave % RW, sx = wave / RW;                        // this wave's 32 rows and stream
+    const uint32_t row = rb * (32 * RW) + 32 * rw + n;               // this lane's query row (within the KV head)
     const bool rlive = row < a.rows;
-    const bool wlive = !SKIP || rb * (32 * NW) + 32 * wave < a.rows;    // uniform: the wave has a live row
+    const bool wlive = !SKIP || rb * (32 * RW) + 32 * rw < a.rows;    // uniform: the wave has a live row
 
     // ---- staging units of this thread: u = tid + NT*i -> tensor u / (64 NBLK) (= (wave + NW*i) / NBLK, uniform),
     // key u / (2 NBLK) & 31, block (u >> 1) & (NBLK - 1), half u & 1; rows past the page's end reload its last row (masked later)
@@ -199,7 +207,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     // the tensor of unit i. With one unit per thread waves 0-3 stage V and waves 4-7 K: V costs the dequantization, and the
     // SIMDs' issue favours the older of its two waves (w and w + 4), so the older one takes it
     auto unit_tensor = [&](int i) { return UPT == 1 ? 1 - wave / NBLK : (wave + NW * i) / NBLK; };
-    MmRaw<FMT> R0[UPT], R1[UPT];                                     // tile t's raw bytes in R(t % PF)
+    MmRaw<FMT> R0[NS][UPT], R1[NS][UPT];                             // step t's raw bytes in R(t % PF)
     uint32_t vo[UPT], vq[UPT];                                       // a unit's scale and value bytes in its tile
     #pragma unroll
     for (int i = 0; i < UPT; i++) {
@@ -227,7 +235,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     // past it read zeros and are masked later). Past the chunk's last tile (live false) the same loads go out with an empty
     // range (no memory access, zeros), so that every step issues the same batch and the wait before a tile's dequant
     // covers its own batch only.
-    auto load_tile = [&](MmRaw<FMT> (&R)[UPT], bool live) {
+    auto load_one = [&](MmRaw<FMT> (&R)[UPT], bool live) {
         if (live && ltl == 0) {
             do { lpg++; lkeys = a.pstart[lpg + 1] - a.pstart[lpg]; } while (lkeys == 0);
             ltl = (lkeys - 1) / 32 + 1;
@@ -250,8 +258,11 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
         lv += rs32;
         ltl -= 1;
     };
-    auto store_tile = [&](const MmRaw<FMT> (&R)[UPT], int stage) {
-        char * st = smem + stage * G::STAGE;
+    auto load_tile = [&](MmRaw<FMT> (&R)[NS][UPT], uint32_t t) {     // step t's tiles NS t .. NS t + NS - 1
+        #pragma unroll
+        for (int x = 0; x < NS; x++) load_one(R[x], NS * t + x < ntiles);
+    };
+    auto store_one = [&](const MmRaw<FMT> (&R)[UPT], char * st) {
         #pragma unroll
         for (int i = 0; i < UPT; i++) {
             const int u = tid + NT * i;
@@ -273,10 +284,15 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
         }
     };
 
+    auto store_tile = [&](const MmRaw<FMT> (&R)[NS][UPT], int stage) {
+        #pragma unroll
+        for (int x = 0; x < NS; x++) store_one(R[x], smem + (stage * NS + x) * G::STAGE);
+    };
+
     // ---- the first two tiles' loads, then the query rows (B operand: lane (h2, n) holds row n, dims 16kk + 8h2 + t)
-    load_tile(R0, true);
+    load_tile(R0, 0);
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (PF == 2) load_tile(R1, ntiles > 1);
+    if constexpr (PF == 2) load_tile(R1, 1);
     __builtin_amdgcn_sched_barrier(0);
     mm_h8 Qf[HD / 16];                                               // !EX: fp16 query operands
     pa_u4 Qi[NBLK];                                                  // EX: int8 query quants per block
@@ -310,7 +326,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
 
     // ---- prologue: tile t0 -> stage 0, tile t0 + 2's loads in flight in R0 (t0 + 1's in R1)
     store_tile(R0, 0);
-    load_tile(R0, ntiles > PF);
+    load_tile(R0, PF);
     mm_lds_barrier();
 
     mm_f16 O[NBLK];
@@ -332,7 +348,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     uint32_t dk2 = 0u;
     auto kf_read = [&](const char * Kt, int kk) { kf[kk % KA] = *(const mm_h8 *) (Kt + n * G::KST + 32 * kk + 16 * h2); };
     auto k_read = [&](int stage) {
-        const char * Kt = smem + stage * G::STAGE;
+        const char * Kt = smem + (stage * NS + sx) * G::STAGE;
         if constexpr (EX) {
             dk2 = *(const uint32_t *) (Kt + G::KT + G::VT + 8 * n + 4 * h2);
             #pragma unroll
@@ -345,7 +361,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     };
     // one tile's matrix work on LDS stage `stage` (nvalid keys)
     auto compute = [&](int stage, int nvalid) {
-        const char * Kt = smem + stage * G::STAGE;
+        const char * Kt = smem + (stage * NS + sx) * G::STAGE;
         const char * Vt = Kt + G::KT;
 
         // V^T per (dim block db, 16-key half mi), idx = 2 db + mi, by two transposing reads (lane 16q + s reads key row 16mi +
@@ -448,36 +464,75 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
         }
     };
     // one tile step; Rn holds tile t + 1's raw bytes
-    auto step = [&](uint32_t t, MmRaw<FMT> (&Rn)[UPT]) {
+    auto step = [&](uint32_t t, MmRaw<FMT> (&Rn)[NS][UPT]) {
         const int stage = t & 1;
-        if (ctl == 0) {                                              // before any LDS operation of this step
-            uint32_t keys;
-            do { cpg++; keys = a.pstart[cpg + 1] - a.pstart[cpg]; } while (keys == 0);
-            ctl = (keys - 1) / 32 + 1;
-            clast = (keys - 1) % 32 + 1;
-            __builtin_amdgcn_s_waitcnt(0xc07f);
+        int nvalid = 0;                                              // keys of this wave's tile (0 past the chunk's end)
+        #pragma unroll
+        for (int x = 0; x < NS; x++) {
+            if (NS > 1 && NS * t + x >= ntiles) break;
+            if (ctl == 0) {                                          // before any LDS operation of this step
+                uint32_t keys;
+                do { cpg++; keys = a.pstart[cpg + 1] - a.pstart[cpg]; } while (keys == 0);
+                ctl = (keys - 1) / 32 + 1;
+                clast = (keys - 1) % 32 + 1;
+                __builtin_amdgcn_s_waitcnt(0xc07f);
+            }
+            const uint32_t nv = ctl == 1 ? clast : 32u;
+            ctl -= 1;
+            if (NS == 1 || x == sx) nvalid = (int) nv;
         }
-        const int nvalid = (int) (ctl == 1 ? clast : 32u);
-        ctl -= 1;
-        // the next tile's bytes -> the other stage (last read before the previous barrier; past the chunk's end the
-        // stage is written and never read), then tile t + 1 + PF's loads into the registers just freed
+        const bool clive = wlive && (NS == 1 || nvalid > 0);
+        // the next step's bytes -> the other stage (last read before the previous barrier; past the chunk's end the
+        // stage is written and never read), then step t + 1 + PF's loads into the registers just freed
         if (KEARLY) k_read(stage);
         store_tile(Rn, stage ^ 1);
-        load_tile(Rn, t + 1 + PF < ntiles);
-        if (wlive) compute(stage, nvalid);
+        load_tile(Rn, t + 1 + PF);
+        if (clive) compute(stage, nvalid);
         mm_lds_barrier();                                            // this stage is free; the next one is written
     };
-    uint32_t t = 0;                                                  // tile t + 1 is in R((t + 1) % PF)
+    const uint32_t nsteps = (ntiles + NS - 1) / NS;
+    uint32_t t = 0;                                                  // step t + 1's tiles are in R((t + 1) % PF)
     if constexpr (PF == 2) {
-        for (; t + 2 <= ntiles; t += 2) {
+        for (; t + 2 <= nsteps; t += 2) {
             step(t, R1);
             step(t + 1, R0);
         }
-        if (t < ntiles) step(t, R1);
+        if (t < nsteps) step(t, R1);
     } else {
-        for (; t < ntiles; t++) step(t, R0);
+        for (; t < nsteps; t++) step(t, R0);
     }
 
+    if constexpr (NS > 1) {
+        // fold the streams: each but the first leaves its rows' O, reference and exact max and sum in the stages (free after
+        // the last barrier), lane by lane; the first one's waves rebase both to the larger reference max and add
+        float * fold = (float *) smem + rw * 67 * 64 + lane;
+        static_assert(RW * 67 * 256 <= 2 * NS * G::STAGE, "the streams fold through the stages");
+        #pragma unroll
+        for (int x = 1; x < NS; x++) {
+            if (sx == x && wlive) {
+                #pragma unroll
+                for (int db = 0; db < NBLK; db++)
+                    #pragma unroll
+                    for (int v = 0; v < 16; v++) fold[64 * (16 * db + v)] = O[db][v];
+                fold[64 * 64] = mref; fold[64 * 65] = mx; fold[64 * 66] = lsum;
+            }
+            mm_lds_barrier();
+            if (sx == 0 && wlive) {
+                const float m1 = fold[64 * 64], mn = fmaxf(mref, m1);
+                const float f0 = mref == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mref - mn);
+                const float f1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - mn);
+                #pragma unroll
+                for (int db = 0; db < NBLK; db++)
+                    #pragma unroll
+                    for (int v = 0; v < 16; v++) O[db][v] = O[db][v] * f0 + fold[64 * (16 * db + v)] * f1;
+                mx = fmaxf(mx, fold[64 * 65]);
+                lsum = lsum * f0 + fold[64 * 66] * f1;
+                mref = mn;
+            }
+            if (x + 1 < NS) mm_lds_barrier();
+        }
+        if (sx != 0) return;
+    }
     mx = mm_max32(mx);                                               // the exact row max, tracked per half row
     mm_write_out<HD>(a, O, mref, mx, lsum, h, row, rlive, h2, c);
 }
@@ -486,11 +541,12 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
 // prefill chunks); the reference engines' rounding (PA_QMODE_F16) and f16 K take the fp16-operand QK, the Metal
 // engine's own arithmetic (K dequantized to half in threadgroup memory, pa-metal.mm:379-487)
 template <int HD, int FMT, bool EX>
-static hipError_t launch_mma_fmt(int nw, bool skip, const AttnArgs & a, uint32_t grid, hipStream_t st, hipEvent_t ev0,
+static hipError_t launch_mma_fmt(int nw, bool skip, int streams, const AttnArgs & a, uint32_t grid, hipStream_t st, hipEvent_t ev0,
                                  hipEvent_t ev1) {
     switch (nw) {
         case 4:
-            if (skip) hipExtLaunchKernelGGL((mma_kernel<HD, FMT, 4, true, EX>), dim3(grid), dim3(256), 0, st, ev0, ev1, 0, a);
+            if (streams == 2) hipExtLaunchKernelGGL((mma_kernel<128, FMT, 4, true, EX, 2>), dim3(grid), dim3(256), 0, st, ev0, ev1, 0, a);
+            else if (skip) hipExtLaunchKernelGGL((mma_kernel<HD, FMT, 4, true, EX>), dim3(grid), dim3(256), 0, st, ev0, ev1, 0, a);
             else hipExtLaunchKernelGGL((mma_kernel<HD, FMT, 4, false, EX>), dim3(grid), dim3(256), 0, st, ev0, ev1, 0, a);
             break;
         case 8:
@@ -502,12 +558,12 @@ static hipError_t launch_mma_fmt(int nw, bool skip, const AttnArgs & a, uint32_t
     return hipGetLastError();
 }
 
-static hipError_t launch_mma_128(int fmt, int nw, bool skip, const AttnArgs & a, uint32_t grid, hipStream_t st, hipEvent_t ev0,
+static hipError_t launch_mma_128(int fmt, int nw, bool skip, int streams, const AttnArgs & a, uint32_t grid, hipStream_t st, hipEvent_t ev0,
                                  hipEvent_t ev1) {
     const bool ex = a.qmode == 0;                                    // PA_QMODE_GGML over quantized K: exact block dots
-    if (fmt == 0) return launch_mma_fmt<128, 0, false>(nw, skip, a, grid, st, ev0, ev1);
-    if (fmt == 1) return ex ? launch_mma_fmt<128, 1, true>(nw, skip, a, grid, st, ev0, ev1) : launch_mma_fmt<128, 1, false>(nw, skip, a, grid, st, ev0, ev1);
-    if (fmt == 2) return ex ? launch_mma_fmt<128, 2, true>(nw, skip, a, grid, st, ev0, ev1) : launch_mma_fmt<128, 2, false>(nw, skip, a, grid, st, ev0, ev1);
+    if (fmt == 0) return launch_mma_fmt<128, 0, false>(nw, skip, streams, a, grid, st, ev0, ev1);
+    if (fmt == 1) return ex ? launch_mma_fmt<128, 1, true>(nw, skip, streams, a, grid, st, ev0, ev1) : launch_mma_fmt<128, 1, false>(nw, skip, streams, a, grid, st, ev0, ev1);
+    if (fmt == 2) return ex ? launch_mma_fmt<128, 2, true>(nw, skip, streams, a, grid, st, ev0, ev1) : launch_mma_fmt<128, 2, false>(nw, skip, streams, a, grid, st, ev0, ev1);
     return hipErrorInvalidValue;
 }
 
@@ -526,9 +582,9 @@ static hipError_t launch_mma_256(int fmt, bool skip, const AttnArgs & a, uint32_
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_mma(int hd, int fmt, int nw, bool skip, const AttnArgs & a, uint32_t grid, hipStream_t st, hipEvent_t ev0,
+hipError_t launch_mma(int hd, int fmt, int nw, bool skip, int streams, const AttnArgs & a, uint32_t grid, hipStream_t st, hipEvent_t ev0,
                       hipEvent_t ev1) {
-    if (hd == 128) return launch_mma_128(fmt, nw, skip, a, grid, st, ev0, ev1);
+    if (hd == 128) return launch_mma_128(fmt, nw, skip, streams, a, grid, st, ev0, ev1);
     if (hd == 256 && nw == 8) return launch_mma_256(fmt, skip, a, grid, st, ev0, ev1);
     return hipErrorInvalidValue;
 }

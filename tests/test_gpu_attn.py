@@ -97,6 +97,21 @@ def test_head256_wide_rows(ws, fmt, rows, workgroups):
         ws.set_split()
 
 
+@pytest.mark.parametrize("qmode", [bb.QMODE_GGML, bb.QMODE_F16])
+@pytest.mark.parametrize("fmt", [bb.FMT_Q8_0, bb.FMT_Q4_0, bb.FMT_F16])
+@pytest.mark.parametrize("rows", [9, 33, 64])
+def test_two_streams(ws, fmt, rows, qmode):
+    """Up to 64 rows over long chunks (two tile streams per workgroup, folded through LDS): chunks of 36 tiles (the last
+    one shorter) and one chunk of all 73, an odd count whose last step has one tile, over pages that end inside a step, hold
+    less than a tile or nothing."""
+    for workgroups in (4, 1):
+        ws.set_split(mma_workgroups=workgroups)
+        try:
+            run_and_check(ws, fmt, 2, rows, 128, 2281, seed=1900 + rows + fmt, qmode=qmode, page_keys=[1000, 7, 0, 64, 1210])
+        finally:
+            ws.set_split()
+
+
 @pytest.mark.parametrize("fmt", [bb.FMT_Q8_0, bb.FMT_F16])
 def test_mma256_split_invariance(ws, fmt):
     """The head-dim-256 kernel at the reference's 48 rows x 4 KV heads over chunks of 1, 2, 3, 5 and 40 tiles and one
