@@ -623,6 +623,28 @@ bool pages_aligned(const char * fn, void * const * kp, void * const * vp, uint32
         }
     return true;
 }
+
+// the launches of a converting APPEND: rows of up to APPEND_SEGS pages each, and at most 2^23 workgroups (2^31 threads);
+// `row` = bytes of a source row, the rest of `a` filled in
+int append_launches(AppendArgs & a, bool from_f32, void * const * kp, void * const * vp, uint32_t page_keys, uint32_t pos0,
+                    const uint8_t * K, const uint8_t * V, size_t row, uint32_t n, hipStream_t st) {
+    const uint64_t max_rows = std::max<uint64_t>(1, (1u << 23) / ((2ull * a.nkv * (a.hd / 32) + 15) / 16));
+    for (uint32_t done = 0; done < n;) {
+        const uint32_t pi = (pos0 + done) / page_keys, off = (pos0 + done) % page_keys;
+        const uint32_t take = (uint32_t) std::min<uint64_t>({n - done, max_rows, (uint64_t) APPEND_SEGS * page_keys - off});
+        a.off0 = off; a.page_keys = page_keys; a.n = take;
+        a.ksrc = K + (size_t) done * row;
+        a.vsrc = V + (size_t) done * row;
+        const uint32_t last = (uint32_t) (((uint64_t) off + take - 1) / page_keys);
+        for (uint32_t i = 0; i < (uint32_t) APPEND_SEGS; i++) {
+            a.kdst[i] = i <= last ? (uint8_t *) kp[pi + i] : nullptr;
+            a.vdst[i] = i <= last ? (uint8_t *) vp[pi + i] : nullptr;
+        }
+        if (!hip_ok(launch_append(from_f32, a, st), from_f32 ? "append quantize launch" : "append f16 launch")) return -1;
+        done += take;
+    }
+    return 0;
+}
 }  // namespace
 
 extern "C" int pa_hip_append_rows(const pa_hip_shape * s, void * const * k_pages, void * const * v_pages, int n_pages,
@@ -634,24 +656,22 @@ extern "C" int pa_hip_append_rows(const pa_hip_shape * s, void * const * k_pages
     if (n > 0 && (!K || !V)) { set_err("pa_hip_append_rows: null K/V"); return -1; }
     if (f16 && !pages_aligned("pa_hip_append_rows", k_pages, v_pages, page_keys, pos0, n, 4)) return -1;
     hipStream_t st = (hipStream_t) stream;
-    for (uint32_t done = 0; done < n;) {
+    if (f16) {
+        AppendArgs a;
+        a.nkv = s->nkv; a.hd = s->hd; a.rs = srs; a.hb = s->hd * 2; a.src_rs = s->rs; a.src_hb = s->hb;
+        a.fmt = PA_FMT_F16;
+        return append_launches(a, false, k_pages, v_pages, page_keys, pos0, (const uint8_t *) K, (const uint8_t *) V, s->rs, n, st);
+    }
+    for (uint32_t done = 0; done < n;) {                              // rows as received: one copy per page segment
         const uint32_t pos = pos0 + done, pi = pos / page_keys, off = pos % page_keys;
         const uint32_t take = std::min(n - done, page_keys - off);
         uint8_t * kd = (uint8_t *) k_pages[pi] + (size_t) off * srs;
         uint8_t * vd = (uint8_t *) v_pages[pi] + (size_t) off * srs;
         const uint8_t * ks = (const uint8_t *) K + (size_t) done * s->rs;
         const uint8_t * vs = (const uint8_t *) V + (size_t) done * s->rs;
-        if (!f16) {                                                   // rows as received: one copy per page segment
-            if (!hip_ok(hipMemcpyAsync(kd, ks, (size_t) take * s->rs, hipMemcpyDefault, st), "hipMemcpyAsync K") ||
-                !hip_ok(hipMemcpyAsync(vd, vs, (size_t) take * s->rs, hipMemcpyDefault, st), "hipMemcpyAsync V"))
-                return -1;
-        } else {
-            AppendArgs a;
-            a.kdst = kd; a.vdst = vd; a.ksrc = ks; a.vsrc = vs;
-            a.n = take; a.nkv = s->nkv; a.hd = s->hd; a.rs = srs; a.hb = s->hd * 2; a.src_rs = s->rs; a.src_hb = s->hb;
-            a.fmt = PA_FMT_F16;
-            if (!hip_ok(launch_append(false, a, st), "append f16 launch")) return -1;
-        }
+        if (!hip_ok(hipMemcpyAsync(kd, ks, (size_t) take * s->rs, hipMemcpyDefault, st), "hipMemcpyAsync K") ||
+            !hip_ok(hipMemcpyAsync(vd, vs, (size_t) take * s->rs, hipMemcpyDefault, st), "hipMemcpyAsync V"))
+            return -1;
         done += take;
     }
     return 0;
@@ -665,21 +685,11 @@ extern "C" int pa_hip_append_f32(const pa_hip_shape * s, void * const * k_pages,
     const uint32_t al = s->fmt == PA_FMT_F16 ? 4 : 2;                // the stores are 32-bit (f16) or 16-bit words
     if (s->rs % al || s->hb % al) { set_err("pa_hip_append_f32: rs and hb must be multiples of " + std::to_string(al)); return -1; }
     if (!pages_aligned("pa_hip_append_f32", k_pages, v_pages, page_keys, pos0, n, al)) return -1;
-    hipStream_t st = (hipStream_t) stream;
-    for (uint32_t done = 0; done < n;) {
-        const uint32_t pos = pos0 + done, pi = pos / page_keys, off = pos % page_keys;
-        const uint32_t take = std::min(n - done, page_keys - off);
-        AppendArgs a;
-        a.kdst = (uint8_t *) k_pages[pi] + (size_t) off * s->rs;
-        a.vdst = (uint8_t *) v_pages[pi] + (size_t) off * s->rs;
-        a.ksrc = K + (size_t) done * s->nkv * s->hd;
-        a.vsrc = V + (size_t) done * s->nkv * s->hd;
-        a.n = take; a.nkv = s->nkv; a.hd = s->hd; a.rs = s->rs; a.hb = s->hb; a.src_rs = 0; a.src_hb = 0;
-        a.fmt = (int) s->fmt;
-        if (!hip_ok(launch_append(true, a, st), "append quantize launch")) return -1;
-        done += take;
-    }
-    return 0;
+    AppendArgs a;
+    a.nkv = s->nkv; a.hd = s->hd; a.rs = s->rs; a.hb = s->hb; a.src_rs = 0; a.src_hb = 0;
+    a.fmt = (int) s->fmt;
+    return append_launches(a, true, k_pages, v_pages, page_keys, pos0, (const uint8_t *) K, (const uint8_t *) V,
+                           (size_t) s->nkv * s->hd * sizeof(float), n, (hipStream_t) stream);
 }
 
 extern "C" int pa_hip_quantize(int fmt, const float * x, void * y, int64_t n, void * stream) {

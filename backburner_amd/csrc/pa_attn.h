@@ -57,10 +57,12 @@ hipError_t launch_mma256(int fmt, bool skip, const AttnArgs & a, uint32_t grid, 
                          hipEvent_t ev1 = nullptr);
 hipError_t launch_quantize(int fmt, const float * x, void * y, int64_t n, hipStream_t st);
 
-struct AppendArgs {                 // one page segment of an APPEND: rows j = 0 .. n-1
-    uint8_t * kdst, * vdst;         // the segment's first row in the K / V page
+constexpr int APPEND_SEGS = 16;     // pages that one append launch touches (their pointers travel in the kernel arguments)
+
+struct AppendArgs {                 // up to APPEND_SEGS page segments of an APPEND: rows j = 0 .. n-1, row j at position
+    uint8_t * kdst[APPEND_SEGS], * vdst[APPEND_SEGS];   // (off0 + j) % page_keys of page (off0 + j) / page_keys
     const void * ksrc, * vsrc;      // fp32 [n][nkv][hd] (append_quant_kernel) or received rows (append_f16_kernel)
-    uint32_t n, nkv, hd;
+    uint32_t n, off0, page_keys, nkv, hd;
     uint32_t rs, hb;                // stored row and head strides (bytes)
     uint32_t src_rs, src_hb;        // received row and head strides (append_f16_kernel)
     int fmt;                        // stored format (append_quant_kernel)

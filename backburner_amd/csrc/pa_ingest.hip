@@ -86,33 +86,50 @@ __global__ __launch_bounds__(256) void quantize_kernel(const float * __restrict_
     quant_block16(fmt, xb[2 * l], xb[2 * l + 1], l, y + b * (fmt == 1 ? 34 : 18));
 }
 
-// block u of the segment -> (tensor K/V, row j, head h, block b); rows j of the segment land at dst + j*rs
+// APPEND: workgroup = 16 consecutive 32-blocks (16 lanes each) of one row's K and V blocks, in the order (tensor, head, block);
+// the row, its page and the row's first block are scalar, so a lane divides by nothing but the power of two hd / 32. One
+// launch covers up to APPEND_SEGS pages. What bounds it: launch and memory latency (512 tokens x 8 heads x 128 move 5.3 MB,
+// 1 us at the copy rate); a launch per page segment and four 32-bit divisions per lane took 7.1 us per call for a chunk over a
+// page boundary, this form 4.6 (one token 4.5); 2,000 tokens x 4 heads x 256 of q4_0 12.1 and 8.0.
+struct AppendAt {                   // this lane's block: its values (row j, head h, block b) and its page bytes
+    bool live;
+    uint32_t tensor, j, h, b;
+    uint8_t * row;                  // the row's first byte in its page
+};
+__device__ __forceinline__ AppendAt append_at(const AppendArgs & a) {
+    AppendAt r;
+    const uint32_t nb = a.hd / 32, lnb = nb == 4 ? 2u : 3u, per_t = a.nkv * nb, wpr = (2 * per_t + 15) / 16;
+    const uint32_t j = blockIdx.x / wpr, q = (blockIdx.x % wpr) * 16 + threadIdx.x / 16;
+    r.live = q < 2 * per_t;                                          // whole 16-lane rows leave together
+    r.tensor = q >= per_t ? 1u : 0u;
+    const uint32_t u = q - r.tensor * per_t;
+    r.j = j;
+    r.h = u >> lnb;
+    r.b = u & (nb - 1);
+    const uint32_t p = a.off0 + j, pg = p / a.page_keys;             // off0 < page_keys: the first segment's offset
+    r.row = (r.tensor ? a.vdst[pg] : a.kdst[pg]) + (size_t) (p - pg * a.page_keys) * a.rs;
+    return r;
+}
+
 __global__ __launch_bounds__(256) void append_quant_kernel(const AppendArgs a) {
-    const uint32_t nb = a.hd / 32, per_t = a.n * a.nkv * nb;
-    const uint32_t t = (blockIdx.x * 256 + threadIdx.x) / 16;
+    const AppendAt t = append_at(a);
     const int l = threadIdx.x % 16;
-    if (t >= 2 * per_t) return;                                      // whole 16-lane rows leave together
-    const uint32_t tensor = t / per_t, u = t % per_t;
-    const uint32_t j = u / (a.nkv * nb), h = (u / nb) % a.nkv, b = u % nb;
-    const float * xb = (const float *) (tensor ? a.vsrc : a.ksrc) + ((size_t) j * a.nkv + h) * a.hd + 32 * b;
+    if (!t.live) return;
+    const float * xb = (const float *) (t.tensor ? a.vsrc : a.ksrc) + ((size_t) t.j * a.nkv + t.h) * a.hd + 32 * t.b;
     const uint32_t bb = a.fmt == 1 ? 34 : a.fmt == 2 ? 18 : 64;
-    uint8_t * o = (tensor ? a.vdst : a.kdst) + (size_t) j * a.rs + (size_t) h * a.hb + (size_t) b * bb;
-    quant_block16(a.fmt, xb[2 * l], xb[2 * l + 1], l, o);
+    quant_block16(a.fmt, xb[2 * l], xb[2 * l + 1], l, t.row + (size_t) t.h * a.hb + (size_t) t.b * bb);
 }
 
 // received q8_0 block -> 32 f16 values f16(d * q) (d * q is exact in fp32, so the one rounding is the reference's);
 // lane l converts quants 2l, 2l+1
 __global__ __launch_bounds__(256) void append_f16_kernel(const AppendArgs a) {
-    const uint32_t nb = a.hd / 32, per_t = a.n * a.nkv * nb;
-    const uint32_t t = (blockIdx.x * 256 + threadIdx.x) / 16;
+    const AppendAt t = append_at(a);
     const int l = threadIdx.x % 16;
-    if (t >= 2 * per_t) return;
-    const uint32_t tensor = t / per_t, u = t % per_t;
-    const uint32_t j = u / (a.nkv * nb), h = (u / nb) % a.nkv, b = u % nb;
-    const uint8_t * blk = (const uint8_t *) (tensor ? a.vsrc : a.ksrc) + (size_t) j * a.src_rs + (size_t) h * a.src_hb + 34 * b;
+    if (!t.live) return;
+    const uint8_t * blk = (const uint8_t *) (t.tensor ? a.vsrc : a.ksrc) + (size_t) t.j * a.src_rs + (size_t) t.h * a.src_hb + 34 * t.b;
     const float d = pa_f16_bits_to_f32((uint16_t) (blk[0] | (blk[1] << 8)));
     const float v0 = d * (float) (int8_t) blk[2 + 2 * l], v1 = d * (float) (int8_t) blk[3 + 2 * l];
-    uint8_t * o = (tensor ? a.vdst : a.kdst) + (size_t) j * a.rs + (size_t) h * a.hb + 64 * (size_t) b;
+    uint8_t * o = t.row + (size_t) t.h * a.hb + 64 * (size_t) t.b;
     const uint32_t h0 = __builtin_bit_cast(uint16_t, (_Float16) v0), h1 = __builtin_bit_cast(uint16_t, (_Float16) v1);
     *(uint32_t *) (o + 4 * l) = h0 | (h1 << 16);
 }
@@ -125,9 +142,9 @@ hipError_t launch_quantize(int fmt, const float * x, void * y, int64_t n, hipStr
 }
 
 hipError_t launch_append(bool from_f32, const AppendArgs & a, hipStream_t st) {
-    const uint64_t threads = 16ull * 2 * a.n * a.nkv * (a.hd / 32);    // 16 lanes per 32-block
-    if (threads == 0) return hipSuccess;
-    const dim3 grid((uint32_t) ((threads + 255) / 256));
+    const uint32_t wpr = (2 * a.nkv * (a.hd / 32) + 15) / 16;        // workgroups per row
+    if (a.n == 0) return hipSuccess;
+    const dim3 grid(a.n * wpr);
     if (from_f32) hipLaunchKernelGGL(append_quant_kernel, grid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL(append_f16_kernel, grid, dim3(256), 0, st, a);
     return hipGetLastError();

@@ -120,6 +120,35 @@ def test_append_f32(fmt, hd):
         pages.close()
 
 
+@pytest.mark.parametrize("nkv,hd,fmt", [(1, 128, bb.FMT_Q8_0), (3, 128, bb.FMT_Q4_0), (5, 256, bb.FMT_F16)])
+def test_append_over_many_pages(nkv, hd, fmt):
+    """One call over more pages than a launch takes (16), from inside a page, with rows whose blocks do not fill whole
+    workgroups: fp32 rows quantized, and received q8_0 rows stored as f16, bit for bit."""
+    page, pos0, n = 3, 2, 61                                             # pages 0 .. 20
+    n_pages = (pos0 + n + page - 1) // page
+    X = orc.normal(31, 0, n * nkv * hd).reshape(n, nkv, hd).astype(np.float32)
+    for store_f16 in (False, True):
+        hb = orc.head_bytes(bb.FMT_Q8_0 if store_f16 else fmt, hd); rs = nkv * hb
+        out_rs = nkv * hd * 2 if store_f16 else rs
+        print(f"append over {n_pages} pages nkv={nkv} hd={hd} fmt={fmt} store_f16={store_f16}", flush=True)
+        pages = bb.alloc_pages(n_pages, page * out_rs)
+        try:
+            if store_f16:
+                rows = orc.rows_from_f32(bb.FMT_Q8_0, X, rs, hb)
+                dR = bb.DeviceBuffer.from_array(rows)
+                bb.append_rows(bb.make_shape(nkv, 8, hd, bb.FMT_Q8_0, rs=rs), pages, page, pos0, dR.ptr, dR.ptr, n, store_f16=True)
+                want = orc.store_rows_f16(rows, n, nkv, hd, rs, hb).view(np.uint8).reshape(-1)
+            else:
+                dX = bb.DeviceBuffer.from_array(X)
+                bb.append_f32(bb.make_shape(nkv, 8, hd, fmt, rs=rs), pages, page, pos0, dX.ptr, dX.ptr, n)
+                want = orc.rows_from_f32(fmt, X, rs, hb)
+            bb.device_sync()
+            for got in page_bytes(pages, n_pages, page * out_rs):
+                assert np.array_equal(got[pos0 * out_rs:(pos0 + n) * out_rs], want)
+        finally:
+            pages.close()
+
+
 def test_append_rejects_positions_past_the_pages():
     shape = bb.make_shape(8, 8, 128, bb.FMT_Q8_0)
     pages = bb.alloc_pages(1, PAGE_KEYS * shape.rs)
