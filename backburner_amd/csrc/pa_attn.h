@@ -78,8 +78,9 @@ hipError_t launch_coattn(int hd, const uint16_t * Oh, const float * lse, const f
 #ifndef PA_ACCEPT_SEG
 #define PA_ACCEPT_SEG 16384
 #endif
-// logits per acceptance workgroup (a multiple of 1024). [17][151936] fp32: 7.2 us at 16384 (170 workgroups), 8.3 at
-// 8192, 8.8 at 32768, 12.0 at 4096 - fewer, fuller workgroups, and fewer keys for the last one to fold
+// logits per acceptance workgroup (a multiple of 1024): fewer, fuller workgroups, and fewer keys for the last one to fold.
+// [17][151936] fp32, kernel time with a 64-bit key per value: 7.2 us at 16384 (170 workgroups), 8.3 at 8192, 8.8 at 32768,
+// 12.0 at 4096
 constexpr int ACCEPT_SEG = PA_ACCEPT_SEG;
 
 struct AcceptArgs {

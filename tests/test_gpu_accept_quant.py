@@ -71,6 +71,26 @@ def test_accept_edge_values(ws):
         assert gpu_accept(ws, lg, dr)[:2] == orc.accept(lg, dr)[:2]
 
 
+@pytest.mark.parametrize("vocab", [1, 3, 4, 255, 1024, 16383, 16384, 16385, 16388, 50001, 50004])
+def test_accept_segment_edges(ws, vocab):
+    """Both load widths around whole segments (16,384 values): the largest value, ties, -0 == +0, NaN of either sign and
+    rows of -inf at the first and last places of a segment, against numpy.argmax."""
+    rng = np.random.default_rng(vocab)
+    at = sorted({0, 1 % vocab, vocab // 2, max(0, vocab - 2), vocab - 1, min(16383, vocab - 1), min(16384, vocab - 1)})
+    rows = [np.full(vocab, -np.inf, np.float32)]
+    for p in at:
+        a = rng.standard_normal(vocab).astype(np.float32); a[p] = 100.0; rows.append(a)
+        a = np.full(vocab, -1.0, np.float32); a[p] = -0.0; a[at[-1]] = 0.0; rows.append(a)
+        a = rng.standard_normal(vocab).astype(np.float32); a[p:] = np.where(rng.random(vocab - p) < 0.5, np.nan, a[p:]); a[p] = -np.nan
+        rows.append(a)
+        a = np.full(vocab, -np.inf, np.float32); a[p] = -3e38; rows.append(a)
+        a = np.full(vocab, np.inf, np.float32); a[:p] = 1.0; rows.append(a)
+    logits = np.stack(rows)
+    print(f"accept edges vocab={vocab} rows={len(rows)}", flush=True)
+    am = gpu_accept(ws, logits, np.zeros(len(rows) - 1, np.int32))[2]
+    assert np.array_equal(am, np.argmax(logits, axis=1))
+
+
 def test_accept_repeated_calls_reset_counter(ws):
     rng = np.random.default_rng(9)
     for it in range(5):
