@@ -1,6 +1,6 @@
 // pa_mma.h - device helpers shared by the matrix-core attention kernels (pa_mma.hip: head dim 128;
 // pa_mma256.hip: head dim 256): raw K/V staging units and their fp16 dequantization, the LDS-only barrier, lane
-// reductions and the scalar page cursor.
+// reductions and wave-uniform values.
 #pragma once
 #include "pa_attn.h"
 #include "pa_common.h"
@@ -27,43 +27,6 @@ template <int FMT> struct MmRaw {
     pa_u4 q[FMT == 0 ? 2 : 1];
     uint32_t d;
 };
-
-// One unit through a buffer resource (the tile's scalar base, its valid bytes as the range) and a 32-bit offset
-template <int FMT>
-__device__ __forceinline__ void mm_load_unit_buf(MmRaw<FMT> & r, __amdgpu_buffer_rsrc_t rsrc, uint32_t off, int half) {
-    if constexpr (FMT == 1) {
-        r.q[0] = __builtin_bit_cast(pa_u4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off + 2 + 16 * half, 0, 0));
-        r.d = __builtin_amdgcn_raw_buffer_load_b16(rsrc, off, 0, 0);
-    } else if constexpr (FMT == 2) {
-        r.q[0] = __builtin_bit_cast(pa_u4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off + 2, 0, 0));
-        r.d = __builtin_amdgcn_raw_buffer_load_b16(rsrc, off, 0, 0);
-    } else {
-        r.q[0] = __builtin_bit_cast(pa_u4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off + 32 * half, 0, 0));
-        r.q[1] = __builtin_bit_cast(pa_u4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off + 32 * half + 16, 0, 0));
-        r.d = 0;
-    }
-}
-
-// The same unit with the quantized formats' 16 value bytes read at an even-aligned address: a 16-byte load at
-// addr & ~2 and a 2-byte load of the unit's last two bytes, joined by byte alignment (q8_0 / q4_0 blocks are 34 / 18
-// bytes, so every other block's values start 2 bytes past a dword boundary, and a 16-byte load there takes the
-// memory pipeline's slow unaligned path). No byte outside the unit is read. base_lo = the low bits of the buffer's
-// base address; any alignment gives the right bytes (an odd one through the slow path).
-template <int FMT>
-__device__ __forceinline__ void mm_load_unit_buf_al(MmRaw<FMT> & r, __amdgpu_buffer_rsrc_t rsrc, uint32_t off, int half,
-                                                    uint32_t base_lo) {
-    if constexpr (FMT == 0) {
-        mm_load_unit_buf<FMT>(r, rsrc, off, half);
-    } else {
-        const uint32_t q = off + 2 + (FMT == 1 ? 16 * half : 0);         // the 16 value bytes
-        const uint32_t sh = (base_lo + q) & 2u;
-        const pa_u4 w = __builtin_bit_cast(pa_u4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, q - sh, 0, 0));
-        const uint32_t t = __builtin_amdgcn_raw_buffer_load_b16(rsrc, q + 14, 0, 0);
-        r.q[0] = (pa_u4){__builtin_amdgcn_alignbyte(w[1], w[0], sh), __builtin_amdgcn_alignbyte(w[2], w[1], sh),
-                         __builtin_amdgcn_alignbyte(w[3], w[2], sh), __builtin_amdgcn_alignbyte(t, w[3], sh)};
-        r.d = __builtin_amdgcn_raw_buffer_load_b16(rsrc, off, 0, 0);
-    }
-}
 
 // 16 values -> fp16 (8 dwords). Quantized formats: byte u (unsigned quant) -> fp16 bits 0x6400 | u = 1024 + u exactly,
 // minus (1024 + bias) exactly, times d (one rounding); with INT the integer quants themselves (exact, no rounding).
@@ -124,27 +87,5 @@ __device__ __forceinline__ const uint8_t * mm_uni(const uint8_t * p) {
     const uint64_t v = (uint64_t) p;
     return (const uint8_t *) (((uint64_t) mm_uni((uint32_t) (v >> 32)) << 32) | mm_uni((uint32_t) v));
 }
-
-// Page cursor (scalar): the page holding a tile, its tile range and key count. A cursor moves only when a tile leaves
-// its page, so the common case reads no kernel argument memory (whose scalar loads would also wait for the LDS
-// operations in flight).
-struct MmCursor {
-    uint32_t pg, tb, te, nk;
-    const uint8_t * kb, * vb;
-    __device__ __forceinline__ void init(const AttnArgs & a) {
-        pg = 0; tb = a.cstart[0]; te = a.cstart[1]; nk = a.pstart[1] - a.pstart[0]; kb = a.kp[0]; vb = a.vp[0];
-    }
-    __device__ __forceinline__ void seek(const AttnArgs & a, uint32_t tau) {
-        while (tau >= te) {
-            pg++;
-            tb = te;
-            te = a.cstart[pg + 1];
-            nk = a.pstart[pg + 1] - a.pstart[pg];
-            kb = a.kp[pg];
-            vb = a.vp[pg];
-            __builtin_amdgcn_s_waitcnt(0xc07f);                      // lgkmcnt(0): no scalar load left outstanding
-        }
-    }
-};
 
 }  // namespace pa_hip

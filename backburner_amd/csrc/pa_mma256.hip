@@ -15,10 +15,16 @@
 //   O^T (16 dims x 16 rows) += V^T . P^T per dim block (16 blocks), one step over the tile's 32 keys taken in the order
 //   the scores sit in (MFMA k index 8g + 4kh + i = key 16kh + 4g + i): the P operand is the lane's own 8 probabilities,
 //   and V^T comes from two transposing reads (ds_read_b64_tr_b16) per dim block.
-// A row's maximum and sum need the 4 lanes n, n + 16, n + 32, n + 48 (two lane swaps). Online softmax in base 2 with a
+// A row's maximum and sum need the 4 lanes n, n + 16, n + 32, n + 48 (two lane swaps, where the reference max moves and at
+// the end: each lane keeps its own). Online softmax in base 2 with a
 // reference max that moves only when a score exceeds it by more than 2^MM_PMAX (O is rescaled rarely); the exact max is
 // tracked beside it. Output: one split-K slot per workgroup (O unnormalised against the base-2 max, max, sum) or the
 // final (O, m, l) when the call has a single chunk.
+//
+// What bounds it: the waves' instruction chains per tile, half of them staging (HBM alone would take 24 us for 48 rows x 4 KV
+// heads x 65,536 q8_0 keys). us per call there, before and after the value bytes were joined at the store instead of the load
+// (whose step then waited for them), addresses came once per page and the lane swaps left the tile loop: 49.1 / 46.2; 6 rows
+// 37.0 / 33.7; 48 rows of q4_0 48.4 / 45.9; 48 rows in ggml's rounding 60.9 / 59.6; 1,536 rows so (16,384 keys) 273 / 266.
 //
 // Reference roles: pa_attn + pa_merge of the Metal engine at this shape (pa-metal.mm:22-131: per (chunk, KV head) a
 // threadgroup of 48 rows dequantizes 32-key K/V blocks into threadgroup memory as half, S = QK^T and O += PV on
@@ -59,9 +65,8 @@ __global__ __launch_bounds__(256, WPS) void mma256_kernel(const AttnArgs a) {
     using G2 = M2Geom<HD>;
     constexpr int NBLK = G2::NBLK, M2_KST = G2::KST, M2_VST = G2::VST, M2_KT = G2::KT, M2_VT = G2::VT;
     constexpr int M2_STAGE = G2::STAGE;
-    // NB tiles' raw bytes are in flight while a tile is computed (a ring of NB register buffers); 3 to 5 measured no
-    // faster than 2 at 48 rows x 4 KV heads x 65k q8_0 keys
-    constexpr int NT = 256, NB = 2;
+    // NB tiles' raw bytes are in flight while a tile is computed (a ring of NB register buffers)
+    constexpr int NT = 256, NB = EX && !SKIP ? 1 : 2;                // (full row blocks of EX: one, the registers of two spill)
     constexpr int UPT = 128 * NBLK / NT;                             // staging units per thread (128 NBLK per tile)
     __shared__ __attribute__((aligned(16))) char smem[2 * M2_STAGE];
 
@@ -71,7 +76,7 @@ __global__ __launch_bounds__(256, WPS) void mma256_kernel(const AttnArgs a) {
     const uint32_t t8 = (a.n_items + 7) / 8;
     const uint32_t w = xcd * t8 + local;
     if (local >= t8 || w >= a.n_items) return;
-    const uint32_t rb = w % a.nrb, h = (w / a.nrb) % a.nkv, c = w / (a.nrb * a.nkv);
+    const uint32_t rb = mm_uni(w % a.nrb), h = mm_uni((w / a.nrb) % a.nkv), c = mm_uni(w / (a.nrb * a.nkv));
     const uint32_t T = a.cstart[a.n_pages];
     const uint32_t t0 = c * a.chunk, ntiles = min(t0 + a.chunk, T) - t0;
 
@@ -82,40 +87,93 @@ __global__ __launch_bounds__(256, WPS) void mma256_kernel(const AttnArgs a) {
     const bool rlive = row < a.rows;
     const bool wlive = !SKIP || rb * 64 + 16 * wave < a.rows;       // uniform: the wave has a live row
 
-    MmCursor cl, cc;
-    cl.init(a); cc.init(a);
-
     // ---- staging units: u = tid + 256 i -> tensor 4 i / NBLK (uniform), key (u / (2 NBLK)) & 31, block (u >> 1) &
     // (NBLK - 1), half u & 1
     using F = MmFmt<FMT>;
     MmRaw<FMT> R[NB][UPT];                                           // tile j's raw bytes in R[j % NB]
-    auto load_tile = [&](MmRaw<FMT> (&Rb)[UPT], uint32_t tau, bool live) {
-        if (live) cl.seek(a, tau);
-        const uint32_t j0 = live ? 32 * (tau - cl.tb) : 0u;
-        const uint32_t last = live ? cl.nk - 1 - j0 : 0u;
-        const uint32_t nrec = live ? min(last + 1, 32u) * a.rs : 0u;   // the tile's rows only (rs < 2^26)
-        #pragma unroll
-        for (int i = 0; i < UPT; i++) {
-            const int u = tid + NT * i;
-            const int tensor = 4 * i / NBLK, key = (u / (2 * NBLK)) & 31, blk = (u >> 1) & (NBLK - 1), half = u & 1;
-            const uint8_t * base = (tensor ? cl.vb : cl.kb) + (size_t) h * a.hb + (size_t) j0 * a.rs;
-            const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *) base, (short) 0, (int) nrec, 0x00020000);
-            mm_load_unit_buf_al<FMT>(Rb[i], rsrc, min((uint32_t) key, last) * a.rs + blk * F::BB, half,
-                                     (uint32_t) (uintptr_t) base);
+    // a unit's bytes in its tile: the scale at vo, the 16 value bytes at vq (f16: 32). The quantized formats' values are read
+    // at an even-aligned address, 16 bytes at va = vq - sh and the last 2 at vq + 14 (their blocks are 34 / 18 bytes, so every
+    // other block's values start 2 bytes past a dword boundary, and a 16-byte load there takes the memory pipeline's slow
+    // unaligned path; any alignment gives the right bytes, an odd one through that path). No byte outside the unit is read.
+    // The two are joined when the tile is stored, not when it is loaded: that waited for the loads in the step that issued
+    // them. va depends on the page's base (32 rows move it by a multiple of 4) and is computed once per page.
+    uint32_t vo[UPT], vq[UPT], va[UPT];
+    #pragma unroll
+    for (int i = 0; i < UPT; i++) {
+        const uint32_t u = tid + NT * i, key = (u / (2 * NBLK)) & 31, blk = (u >> 1) & (NBLK - 1), half = u & 1;
+        vo[i] = key * a.rs + blk * F::BB;
+        vq[i] = vo[i] + (FMT == 1 ? 2 + 16 * half : FMT == 2 ? 2 : 32 * half);
+        va[i] = vq[i];
+    }
+    const int half = tid & 1;
+    uint32_t Rt[NB][UPT], pk[NB], pv[NB];                            // the units' last 2 bytes; their pages' base addresses
+    // ---- page cursors (scalar), as in mma_kernel
+    uint32_t lpg = 0;
+    if (a.ptl < 32u) lpg = min(t0 >> a.ptl, a.n_pages - 1);
+    else while (t0 >= a.cstart[lpg + 1]) lpg++;
+    lpg = mm_uni(lpg);
+    const uint32_t j00 = 32 * (t0 - a.cstart[lpg]);
+    uint32_t lkeys = mm_uni(a.pstart[lpg + 1] - a.pstart[lpg]), ltl = (lkeys - 1) / 32 + 1 - j00 / 32, llast = (lkeys - 1) % 32 + 1;
+    const size_t hoff = (size_t) h * a.hb;
+    const uint8_t * lk = mm_uni(a.kp[lpg] + hoff + (size_t) j00 * a.rs), * lv = mm_uni(a.vp[lpg] + hoff + (size_t) j00 * a.rs);
+    uint32_t cpg = lpg, ctl = ltl, clast = llast;
+    const uint32_t rs32 = 32 * a.rs;
+    auto align_page = [&]() {
+        if constexpr (FMT != 0) {
+            #pragma unroll
+            for (int i = 0; i < UPT; i++) va[i] = vq[i] - (((uint32_t) (uintptr_t) (4 * i / NBLK ? lv : lk) + vq[i]) & 2u);
         }
     };
-    auto store_tile = [&](const MmRaw<FMT> (&Rb)[UPT], int stage) {
+    align_page();
+    auto load_tile = [&](int r, bool live) {
+        if (live && ltl == 0) {
+            do { lpg++; lkeys = a.pstart[lpg + 1] - a.pstart[lpg]; } while (lkeys == 0);
+            ltl = (lkeys - 1) / 32 + 1;
+            llast = (lkeys - 1) % 32 + 1;
+            lk = mm_uni(a.kp[lpg] + hoff);
+            lv = mm_uni(a.vp[lpg] + hoff);
+            __builtin_amdgcn_s_waitcnt(0xc07f);                      // lgkmcnt(0): no scalar load left outstanding
+            align_page();
+        }
+        const uint32_t nrec = (live ? (ltl == 1 ? llast : 32u) : 0u) * a.rs;   // the tile's rows only (rs < 2^26)
+        #pragma unroll
+        for (int i = 0; i < UPT; i++) {
+            const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *) (4 * i / NBLK ? lv : lk), (short) 0, (int) nrec, 0x00020000);
+            if constexpr (FMT == 0) {
+                R[r][i].q[0] = __builtin_bit_cast(pa_u4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, vq[i], 0, 0));
+                R[r][i].q[1] = __builtin_bit_cast(pa_u4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, vq[i] + 16, 0, 0));
+                R[r][i].d = 0;
+            } else {
+                R[r][i].q[0] = __builtin_bit_cast(pa_u4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, va[i], 0, 0));
+                Rt[r][i] = __builtin_amdgcn_raw_buffer_load_b16(rsrc, vq[i] + 14, 0, 0);
+                R[r][i].d = __builtin_amdgcn_raw_buffer_load_b16(rsrc, vo[i], 0, 0);
+            }
+        }
+        pk[r] = (uint32_t) (uintptr_t) lk;
+        pv[r] = (uint32_t) (uintptr_t) lv;
+        lk += rs32;
+        lv += rs32;
+        ltl -= 1;
+    };
+    auto store_tile = [&](int r, int stage) {
         char * st = smem + stage * M2_STAGE;
         #pragma unroll
         for (int i = 0; i < UPT; i++) {
             const int u = tid + NT * i;
-            const int tensor = 4 * i / NBLK, key = (u / (2 * NBLK)) & 31, blk = (u >> 1) & (NBLK - 1), half = u & 1;
+            const int tensor = 4 * i / NBLK, key = (u / (2 * NBLK)) & 31, blk = (u >> 1) & (NBLK - 1);
+            MmRaw<FMT> x = R[r][i];
+            if constexpr (FMT != 0) {
+                const uint32_t sh = ((tensor ? pv[r] : pk[r]) + vq[i]) & 2u;
+                const pa_u4 w = x.q[0];
+                x.q[0] = (pa_u4){__builtin_amdgcn_alignbyte(w[1], w[0], sh), __builtin_amdgcn_alignbyte(w[2], w[1], sh),
+                                 __builtin_amdgcn_alignbyte(w[3], w[2], sh), __builtin_amdgcn_alignbyte(Rt[r][i], w[3], sh)};
+            }
             pa_u4 lo, hi;
             if (EX && tensor == 0) {                                 // K: integer quants, the block scale beside the tile
-                mm_dequant<FMT, true>(Rb[i], half, lo, hi);
-                if (half == 0) *(uint16_t *) (st + M2_KT + M2_VT + 2 * NBLK * key + 2 * blk) = (uint16_t) Rb[i].d;
+                mm_dequant<FMT, true>(x, half, lo, hi);
+                if (half == 0) *(uint16_t *) (st + M2_KT + M2_VT + 2 * NBLK * key + 2 * blk) = (uint16_t) x.d;
             } else {
-                mm_dequant<FMT>(Rb[i], half, lo, hi);
+                mm_dequant<FMT>(x, half, lo, hi);
             }
             char * dst = (tensor ? st + M2_KT + key * M2_VST : st + key * M2_KST) + 2 * (32 * blk + 16 * half);
             *(pa_u4 *) dst = lo;
@@ -125,7 +183,7 @@ __global__ __launch_bounds__(256, WPS) void mma256_kernel(const AttnArgs a) {
 
     #pragma unroll
     for (int i = 0; i < NB; i++) {
-        load_tile(R[i], t0 + i, i == 0 || ntiles > (uint32_t) i);
+        load_tile(i, i == 0 || ntiles > (uint32_t) i);
         __builtin_amdgcn_sched_barrier(0);
     }
 
@@ -173,8 +231,8 @@ __global__ __launch_bounds__(256, WPS) void mma256_kernel(const AttnArgs a) {
         }
     }
 
-    store_tile(R[0], 0);
-    load_tile(R[0], t0 + NB, ntiles > NB);
+    store_tile(0, 0);
+    load_tile(0, ntiles > NB);
     mm_lds_barrier();
 
     pa_f4 O[HD / 16];
@@ -244,9 +302,9 @@ __global__ __launch_bounds__(256, WPS) void mma256_kernel(const AttnArgs a) {
                     if (16 * kh + 4 * g + i >= nvalid) S[kh][i] = -INFINITY;
         }
         float tm = fmaxf(fmaxf(fmaxf(S[0][0], S[0][1]), fmaxf(S[0][2], S[0][3])), fmaxf(fmaxf(S[1][0], S[1][1]), fmaxf(S[1][2], S[1][3])));
-        tm = EX ? mm_max32(m2_max16(tm)) + mc : mm_max32(m2_max16(tm)) * sm;   // row n's tile max, base 2
+        tm = EX ? tm + mc : tm * sm;                                 // this lane's quarter of row n's tile max, base 2
         if (__builtin_amdgcn_ballot_w64(tm > mref + MM_PMAX)) {
-            const float mn = fmaxf(mref, tm);
+            const float mn = fmaxf(mref, mm_max32(m2_max16(tm)));    // the row's other keys: lanes n + 16 i
             const float alpha = mref == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mref - mn);
             #pragma unroll
             for (int db = 0; db < HD / 16; db++) O[db] *= alpha;
@@ -284,27 +342,32 @@ __global__ __launch_bounds__(256, WPS) void mma256_kernel(const AttnArgs a) {
             O[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, P, O[db], 0, 0, 0);
         }
     };
-    auto step = [&](uint32_t t, MmRaw<FMT> (&Rn)[UPT]) {
+    auto step = [&](uint32_t t, int r) {
         const int stage = t & 1;
-        const uint32_t tau = t0 + t, tn = tau + 1 + NB;              // this tile; the one loaded now
-        cc.seek(a, tau);
-        const int nvalid = (int) min(32u, cc.nk - 32 * (tau - cc.tb));
-        const bool nlive = t + 1 + NB < ntiles;
-        if (nlive) cl.seek(a, tn);
-        store_tile(Rn, stage ^ 1);
-        load_tile(Rn, tn, nlive);
+        if (ctl == 0) {                                              // before any LDS operation of this step
+            uint32_t keys;
+            do { cpg++; keys = a.pstart[cpg + 1] - a.pstart[cpg]; } while (keys == 0);
+            ctl = (keys - 1) / 32 + 1;
+            clast = (keys - 1) % 32 + 1;
+            __builtin_amdgcn_s_waitcnt(0xc07f);
+        }
+        const int nvalid = (int) (ctl == 1 ? clast : 32u);
+        ctl -= 1;
+        store_tile(r, stage ^ 1);
+        load_tile(r, t + 1 + NB < ntiles);
         if (wlive) compute(stage, nvalid);
         mm_lds_barrier();
     };
     uint32_t t = 0;                                                  // tile t + 1 is in R[(t + 1) % NB]
     for (; t + NB <= ntiles; t += NB) {
         #pragma unroll
-        for (int k = 0; k < NB; k++) step(t + k, R[(k + 1) % NB]);
+        for (int k = 0; k < NB; k++) step(t + k, (k + 1) % NB);
     }
     #pragma unroll
     for (int k = 0; k < NB - 1; k++)
-        if (t + k < ntiles) step(t + k, R[(k + 1) % NB]);
+        if (t + k < ntiles) step(t + k, (k + 1) % NB);
 
+    mx = mm_max32(m2_max16(mx));                                     // the exact row max, tracked per quarter row
     // ---- row n's result: sum over its 4 lanes, O rebased from the reference max to the exact one
     const float lt = mm_sum32(m2_sum16(lsum));
     const float f = mref == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mref - mx);
