@@ -193,6 +193,10 @@ namespace {
 // round and are slower). q4_0, twice the work per byte: four per CU (45.4-46.4 against 49.5-50.2 us at three).
 constexpr int DEC_TARGET_WG_Q8 = 768, DEC_TARGET_WG_Q4 = 1024;
 
+// The split of the matrix-core kernels (attn_mma): what a step of one tile costs (head dim 128, head dim 256, and there with
+// the exact block dots), the rate at which slots are written and read back, and the merge's launch
+constexpr double TILE_US_128 = 1.5, TILE_US_256 = 2.4, TILE_US_256_EX = 3.0, SLOT_BYTES_PER_US = 4.5e6, MERGE_US = 4.0;
+
 // One call of the engine path: where its split-K slots go, its geometry overrides, its timing events and, for
 // pa_hip_attn_reply, the reply target the merge writes instead of (O, m, l).
 struct Call {
@@ -341,18 +345,24 @@ int attn_decode(Call & cx, const pa_hip_shape * s, const void * const * k_pages,
 }
 
 // the matrix-core kernels, over chunks of 32-key tiles: mma_kernel (row blocks of 32*NW rows) for every head-dim-128 call
-// that attn_decode does not take and for head dim 256 above 64 rows with fp16 operands; mma256_kernel (row blocks of 64
-// rows) for the other head-dim-256 calls
+// that attn_decode does not take and for long head-dim-256 contexts above 64 rows; mma256_kernel (row blocks of 64 rows) for
+// the other head-dim-256 calls
 int attn_mma(Call & cx, const pa_hip_shape * s, const void * const * k_pages, const void * const * v_pages,
              const uint32_t * nkeys, int n_pages, const float * Q, float * O, float * m, float * l, hipStream_t st) {
     // mma_kernel: 32 rows per wave, 8 waves above 128 rows (prefill) and at head dim 256, 4 otherwise (verify, short verify
     // blocks, f16 decode). mma256_kernel: 16 rows per wave, 4 waves (the reference's 48 rows per KV head fill three).
-    // Head dim 256 changes over where a second 64-row block would begin: each 16-row wave reads a whole tile from LDS for
-    // half the rows, and each 64-row block dequantizes it again. us per call, mma256_kernel against mma_kernel: 96 rows x
-    // 65,536 q8_0 keys 81 / 56, 192 rows x 32,768 q4_0 keys 68 / 55, 288 rows x 32,768 q8_0 keys (a second block of one
-    // wave) 99 / 89, 1,536 rows x 16,384 q4_0 keys 211 / 136; 48 rows stay (one 64-row block at two workgroups per CU, 49).
-    // The exact block dots (ggml's rounding over quantized K) need more registers there than 32 rows leave and stay too.
-    const bool h256 = s->hd == 256 && (s->rows <= 64 || (s->qmode == PA_QMODE_GGML && s->fmt != PA_FMT_F16));
+    // Head dim 256 above 64 rows: each 16-row wave reads a whole tile from LDS for half the rows and each 64-row block
+    // dequantizes it again, but an 8-wave workgroup starts and ends 8-10 us later, so mma_kernel is taken for long contexts,
+    // the more rows the sooner. us per call, mma256_kernel against mma_kernel, fp16 operands: 16,384 q8_0 keys, 72 rows 33.0 /
+    // 26.5, 300 rows 58.1 / 56.3, 512 rows 76.7 / 77.4, 900 rows 129.7 / 99.3; 4,096 keys, 72 rows 21.1 / 22.2, 300 rows 34.9
+    // / 40.8, 900 rows 49.0 / 49.4; 1,000 keys, 300 rows 20.8 / 32.1. Exact block dots (ggml's rounding over quantized K),
+    // whose 32-row form converts and scales each dot in vector instructions: 16,384 keys, 192 rows 54.0 / 64.4, 512 rows 99.3 /
+    // 100.1, 600 rows 128.5 / 115.6, 900 rows 174 / 135; 4,096 keys, 900 rows 61 / 68.
+    uint64_t call_tiles = 0;
+    for (int i = 0; i < n_pages; i++) call_tiles += (nkeys[i] + 31ull) / 32;
+    const bool ex = s->qmode == PA_QMODE_GGML && s->fmt != PA_FMT_F16;
+    const bool wide = s->rows > 64 && (ex ? s->rows > 512 && call_tiles >= 384 : std::max(512u, s->rows) * call_tiles >= 512u * 384u);
+    const bool h256 = s->hd == 256 && !wide;
     const uint32_t nw = h256 ? 4u : s->rows > 128 || s->hd == 256 ? 8u : 4u, rpw = h256 ? 16u : 32u;
     const uint32_t nrb = (s->rows + rpw * nw - 1) / (rpw * nw);
     // rows per KV head in the slots: whole row blocks, at head dim 256 multiples of 64 under either kernel (only real rows
@@ -366,8 +376,24 @@ int attn_mma(Call & cx, const pa_hip_shape * s, const void * const * k_pages, co
     // key chunks: by default one round of resident workgroups (one of 8 waves or two of 4 per CU, 256 CUs); a second,
     // partial round costs more than the extra slots save
     const uint64_t target = cx.mma_workgroups > 0 ? (uint64_t) cx.mma_workgroups : 256u * 8 / nw;
+    // fewer chunks where a short context does not pay for them: n chunks take tiles / n steps, and their slots are written
+    // and read again, so the cost is least at n = the root of tiles x tile time / slot time; one chunk, written directly, where
+    // that costs no more than the merge's launch on top. us per call with one round of workgroups whatever the context and
+    // so: 8 heads x 128 rows at head dim 128 over 1,000 f16 keys 19.5 / 14.3, over 4,096 25.7 / 20.0; 4,000 rows over 300 q8_0
+    // keys 34.6 / 25.5, over 1,000 48.9 / 45.0; 4 heads x 48 rows at head dim 256 over 4,096 q8_0 keys 25.8 / 18.6, 300 rows
+    // over 1,000 27.1 / 20.8; from 16,384 keys on the count is one round's again.
+    auto pays = [&](uint64_t tiles) -> uint64_t {
+        const double tile_us = s->hd == 128 ? TILE_US_128 : ex ? TILE_US_256_EX : TILE_US_256;
+        const double slot_us = 2.0 * s->nkv * s->rows * (s->hd * sizeof(float) + sizeof(float2)) / SLOT_BYTES_PER_US;
+        // tiles per chunk: the better of the two counts around the root
+        auto cost = [&](uint64_t t) { return t * tile_us + (tiles + t - 1) / t * slot_us; };
+        uint64_t t = std::max<uint64_t>(1, (uint64_t) std::sqrt(tiles * slot_us / tile_us));
+        if (cost(t + 1) < cost(t)) t++;
+        return tiles * tile_us <= cost(t) + MERGE_US ? 1 : (tiles + t - 1) / t;
+    };
     auto chunking = [&](uint64_t tiles, uint64_t cap, uint32_t & tpc) {
-        const uint64_t want = std::max<uint64_t>(1, std::min(target / units, cap));
+        uint64_t want = std::max<uint64_t>(1, std::min(target / units, cap));
+        if (cx.mma_workgroups == 0) want = std::min(want, pays(tiles));
         tpc = (uint32_t) ((tiles + want - 1) / want);
         if (cx.chunk_keys > 0 && cx.mma_workgroups == 0)             // keys per chunk asked for, within the slot cap
             tpc = (uint32_t) std::max<uint64_t>((tiles + std::min(cap, tiles) - 1) / std::min(cap, tiles),
@@ -384,7 +410,22 @@ int attn_mma(Call & cx, const pa_hip_shape * s, const void * const * k_pages, co
         for_launches(nkeys, n_pages, [&](int, int, uint64_t tiles, uint64_t) { n_slots += chunking(tiles, cap, tpc); });
     }
     const bool direct = n_launch == 1 && n_slots == 1;
-    if (!direct && !cx.slots(n_slots * rows_per_slot, s->hd, st)) return -1;
+    // a workspace gets room for one round of workgroups of either kernel whatever this context pays for, so that a call over
+    // more keys does not have to grow it (which a stream capture refuses)
+    uint64_t room = direct ? 0 : n_slots * rows_per_slot;
+    if (!cx.fixed && cx.mma_workgroups == 0 && cx.chunk_keys == 0) {
+        auto round_rows = [&](uint32_t block, uint64_t workgroups, uint64_t tiles) {
+            const uint64_t n = std::max<uint64_t>(1, workgroups / ((uint64_t) s->nkv * ((s->rows + block - 1) / block)));
+            return std::min(n, tiles) * rows_per_slot;
+        };
+        uint64_t rows = 0;
+        for_launches(nkeys, n_pages, [&](int, int, uint64_t tiles, uint64_t) {
+            rows += s->hd == 256 ? std::max(round_rows(64, 512, tiles), s->rows > 64 ? round_rows(256, 256, tiles) : 0)
+                                 : round_rows(rpw * nw, 2048 / nw, tiles);
+        });
+        if (rows > rows_per_slot) room = std::max(room, rows);
+    }
+    if (room > 0 && !cx.slots(room, s->hd, st)) return -1;
     uint32_t li = 0, slot0 = 0;
     bool ok = true;
     for_launches(nkeys, n_pages, [&](int p0, int np, uint64_t tiles, uint64_t) {

@@ -1,6 +1,6 @@
 // pa_mma.hip - partial attention for many query rows per KV head (16-token verify, 512-token prefill chunks, and any
-// shape with more than 8 rows) over q8_0 / q4_0 / f16 K and V, head dim 128 (and 256 above 64 rows with fp16 operands), on
-// the matrix cores (gfx950).
+// shape with more than 8 rows) over q8_0 / q4_0 / f16 K and V, head dim 128 (and 256 for long contexts above 64 rows),
+// on the matrix cores (gfx950).
 //
 // One workgroup = one KV head x one block of 32*NW query rows x one chunk of consecutive 32-key tiles; NW waves, 32
 // rows each. Per tile the workgroup dequantizes V once into LDS as fp16 (d*q rounded once: the quants become fp16
@@ -44,7 +44,7 @@ namespace pa_hip {
 template <int HD> struct MmGeom {
     static constexpr int NBLK = HD / 32;                      // quant blocks per head row
     static constexpr int KST = 2 * HD + 16, KST8 = HD + 16, VST = 2 * HD + 64;
-    static constexpr int KT = 32 * KST, VT = 32 * VST, KSC = 32 * 2 * NBLK;
+    static constexpr int KT = 32 * KST, VT = 32 * VST, KSC = 32 * NBLK * (HD == 128 ? 2 : 4);
     static constexpr int STAGE = KT + VT + KSC;
 };
 
@@ -95,7 +95,8 @@ __device__ __forceinline__ void mm_prep_qi8(const AttnArgs & a, uint32_t h, uint
         const float id = d != 0.0f ? 1.0f / d : 0.0f;
         const float dq = (float) (_Float16) d * (scale * MM_LOG2E);   // the fp16 block scale * scale, base-2 units
         const _Float16 hi = (_Float16) dq, lo = (_Float16) (dq - (float) hi);
-        dqb[b] = (uint32_t) __builtin_bit_cast(uint16_t, hi) | ((uint32_t) __builtin_bit_cast(uint16_t, lo) << 16);
+        if constexpr (HD == 256) dqb[b] = __builtin_bit_cast(uint32_t, dq * (FMT == 2 ? 0.0625f : 1.0f));
+        else dqb[b] = (uint32_t) __builtin_bit_cast(uint16_t, hi) | ((uint32_t) __builtin_bit_cast(uint16_t, lo) << 16);
         uint32_t w[4];
         int qs = 0;
         #pragma unroll
@@ -110,7 +111,7 @@ __device__ __forceinline__ void mm_prep_qi8(const AttnArgs & a, uint32_t h, uint
             w[j] = v;
         }
         Qi[b] = (pa_u4){w[0], w[1], w[2], w[3]};
-        if constexpr (FMT == 2) {
+        if constexpr (FMT == 2 && HD == 128) {
             const auto t = __builtin_amdgcn_permlane32_swap((unsigned) qs, (unsigned) qs, false, false);
             const int qsum = (int) t[0] + (int) t[1];                // the block's 32 quants: lanes l and l ^ 32
             const float c = (float) (-8 * qsum) * ((float) hi + (float) lo);
@@ -170,7 +171,7 @@ __device__ __forceinline__ void mm_write_out(const AttnArgs & a, const mm_f16 (&
 // q4_0 keys 36.8 / 34.0, 48 rows x 65,536 q4_0 keys (fp16 operands) 45.6 / 43.6.
 template <int HD, int FMT, int NW, bool SKIP, bool EX, int NS = 1>
 __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) {   // 2 waves per SIMD
-    static_assert(!EX || (FMT != 0 && HD == 128), "the exact block dots take quantized K at head dim 128");
+    static_assert(!EX || FMT != 0, "the exact block dots take quantized K");
     using G = MmGeom<HD>;
     constexpr int NBLK = G::NBLK;
     // tiles whose raw bytes are in flight in registers (head dim 256: one; O and Q take 192 of the 256 registers there, and
@@ -201,12 +202,13 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     const bool rlive = row < a.rows;
     const bool wlive = !SKIP || rb * (32 * RW) + 32 * rw < a.rows;    // uniform: the wave has a live row
 
-    // ---- staging units of this thread: u = tid + NT*i -> tensor u / (64 NBLK) (= (wave + NW*i) / NBLK, uniform),
+    // ---- staging units of this thread: u = tid + NT*i -> tensor u / (64 NBLK) (uniform),
     // key u / (2 NBLK) & 31, block (u >> 1) & (NBLK - 1), half u & 1; rows past the page's end reload its last row (masked later)
     using F = MmFmt<FMT>;
     // the tensor of unit i. With one unit per thread waves 0-3 stage V and waves 4-7 K: V costs the dequantization, and the
     // SIMDs' issue favours the older of its two waves (w and w + 4), so the older one takes it
-    auto unit_tensor = [&](int i) { return UPT == 1 ? 1 - wave / NBLK : (wave + NW * i) / NBLK; };
+    static_assert(UPT == 1 || NW == NBLK, "a unit's tensor is then its index, known to the compiler");
+    auto unit_tensor = [&](int i) { return UPT == 1 ? 1 - wave / NBLK : i; };
     MmRaw<FMT> R0[NS][UPT], R1[NS][UPT];                             // step t's raw bytes in R(t % PF)
     uint32_t vo[UPT], vq[UPT];                                       // a unit's scale and value bytes in its tile
     #pragma unroll
@@ -270,9 +272,14 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
             pa_u4 lo, hi;
             if (EX && tensor == 0) {                                 // K: the raw int8 quants (q4_0: this half's
                                                                      // nibbles as unsigned bytes), the block scale beside
-                if (half == 0) *(uint16_t *) (st + G::KT + G::VT + 2 * NBLK * key + 2 * blk) = (uint16_t) R[i].d;
                 pa_u4 q = R[i].q[0];
-                if constexpr (FMT == 2) q = (q >> (4 * half)) & 0x0f0f0f0fu;
+                if constexpr (HD == 128) {
+                    if (half == 0) *(uint16_t *) (st + G::KT + G::VT + 2 * NBLK * key + 2 * blk) = (uint16_t) R[i].d;
+                    if constexpr (FMT == 2) q = (q >> (4 * half)) & 0x0f0f0f0fu;
+                } else {
+                    if (half == 0) *(float *) (st + G::KT + G::VT + 4 * (32 * blk + key)) = pa_f16_bits_to_f32((uint16_t) R[i].d);
+                    if constexpr (FMT == 2) q = ((q << (4 - 4 * half)) & 0xf0f0f0f0u) ^ 0x80808080u;
+                }
                 *(pa_u4 *) (st + key * G::KST8 + 32 * blk + 16 * half) = q;
                 continue;
             }
@@ -304,9 +311,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     // EX: the B operands of the scale products. All four products share one A operand, key n's block scales at k = 2b and
     // 2b + 1 (lanes h2 = b / 2, register b % 2), so block b's B operand holds row n's (hi, lo) pair there, zero elsewhere
     // (one operand per block in otherwise zero registers took four permutes, four selects and eleven moves per tile more)
-    pa_u2 dqw[NBLK];
+    pa_u2 dqw[4];
     #pragma unroll
-    for (int b = 0; b < NBLK; b++) {
+    for (int b = 0; b < 4; b++) {
         const uint32_t x = h2 == (b >> 1) ? dqb[b] : 0u;
         dqw[b] = (b & 1) ? (pa_u2){0u, x} : (pa_u2){x, 0u};
     }
@@ -322,7 +329,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     mm_i16 cvt0;
     #pragma unroll
     for (int v = 0; v < 16; v++) cvt0[v] = 0x4B400000;
-    if constexpr (EX) asm volatile("" : "+v"(cvt0));         // kept in registers, not rebuilt for every tile
+    if constexpr (EX && HD == 128) asm volatile("" : "+v"(cvt0));         // kept in registers, not rebuilt for every tile
 
     // ---- prologue: tile t0 -> stage 0, tile t0 + 2's loads in flight in R0 (t0 + 1's in R1)
     store_tile(R0, 0);
@@ -350,9 +357,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     auto k_read = [&](int stage) {
         const char * Kt = smem + (stage * NS + sx) * G::STAGE;
         if constexpr (EX) {
-            dk2 = *(const uint32_t *) (Kt + G::KT + G::VT + 8 * n + 4 * h2);
+            if constexpr (HD == 128) dk2 = *(const uint32_t *) (Kt + G::KT + G::VT + 8 * n + 4 * h2);
             #pragma unroll
-            for (int b = 0; b < 4; b++) kq[b] = *(const pa_u4 *) (Kt + n * G::KST8 + 32 * b + 16 * h2);
+            for (int b = 0; b < (HD == 128 ? 4 : 2); b++) kq[b] = *(const pa_u4 *) (Kt + n * G::KST8 + 32 * b + 16 * h2);
         } else {
             #pragma unroll
             for (int kk = 0; kk < KA; kk++) kf_read(Kt, kk);
@@ -378,7 +385,26 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
             const pa_h4 x1 = __builtin_bit_cast(pa_h4, __builtin_amdgcn_ds_read_tr16_b64_v4f16((MM_LDS mm_tr4 *) (vb + 8 * G::VST)));
             va[idx % VA] = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
         };
-        if constexpr (EX) {
+        if constexpr (EX && HD == 256) {
+            // per block: the integer dot, then dot * dq_b(row) * dk_b(key) in fp32, the scales of this lane's 16 keys read from
+            // the tile (in fp32, four keys per read): no registers for a scale product or a start value here. q4_0 quants
+            // are staged as 16 (n - 8), their byte's high nibble, and dq_b is divided by 16.
+            #pragma unroll
+            for (int b = 0; b < NBLK; b++) {
+                pa_f4 dk[4];
+                #pragma unroll
+                for (int j = 0; j < 4; j++) dk[j] = *(const pa_f4 *) (Kt + G::KT + G::VT + 4 * (32 * b + 8 * j + 4 * h2));
+                const mm_i16 T = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(mm_i4, kq[b & 1]), __builtin_bit_cast(mm_i4, Qi[b]),
+                                                                     (mm_i16){}, 0, 0, 0);
+                if (b + 2 < NBLK) kq[b & 1] = *(const pa_u4 *) (Kt + n * G::KST8 + 32 * (b + 2) + 16 * h2);
+                const float dq = __builtin_bit_cast(float, dqb[b]);
+                #pragma unroll
+                for (int v = 0; v < 16; v++) S[v] = fmaf((float) T[v] * dq, dk[v / 4][v % 4], b == 0 ? -mc : S[v]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            #pragma unroll
+            for (int i = 0; i < VA; i++) v_read(i);
+        } else if constexpr (EX) {
             // per block: the integer dot on the int8 matrix cores (A: key n's quants, dims 32b + 16h2 .. +15, read raw
             // from the tile; B: the query quants), the scale product, and dot * product summed in fp32
             const pa_u2 dkw = {pa_perm(0u, dk2, 0x01000100u), pa_perm(0u, dk2, 0x03020302u)};
@@ -427,7 +453,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
         if (__builtin_amdgcn_ballot_w64(tm > mref + MM_PMAX)) {
             // rare: move the reference max of every row that needs it (uniform branch)
             float mn = fmaxf(mref, mm_max32(tm));                    // the row's other half: lane ^ 32
-            if constexpr (EX && FMT == 2) {                          // a value the (hi, lo) pair of -mn holds exactly
+            if constexpr (EX && FMT == 2 && HD == 128) {             // a value the (hi, lo) pair of -mn holds exactly
                 const _Float16 mh = (_Float16) mn, ml = (_Float16) (mn - (float) mh);
                 mn = (float) mh + (float) ml;
                 const _Float16 nh = -mh, nl = -ml;
@@ -567,18 +593,18 @@ static hipError_t launch_mma_128(int fmt, int nw, bool skip, int streams, const 
     return hipErrorInvalidValue;
 }
 
-template <int FMT>
+template <int FMT, bool EX>
 static hipError_t launch_mma_256_fmt(bool skip, const AttnArgs & a, uint32_t grid, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
-    if (skip) hipExtLaunchKernelGGL((mma_kernel<256, FMT, 8, true, false>), dim3(grid), dim3(512), 0, st, ev0, ev1, 0, a);
-    else hipExtLaunchKernelGGL((mma_kernel<256, FMT, 8, false, false>), dim3(grid), dim3(512), 0, st, ev0, ev1, 0, a);
+    if (skip) hipExtLaunchKernelGGL((mma_kernel<256, FMT, 8, true, EX>), dim3(grid), dim3(512), 0, st, ev0, ev1, 0, a);
+    else hipExtLaunchKernelGGL((mma_kernel<256, FMT, 8, false, EX>), dim3(grid), dim3(512), 0, st, ev0, ev1, 0, a);
     return hipGetLastError();
 }
 
 static hipError_t launch_mma_256(int fmt, bool skip, const AttnArgs & a, uint32_t grid, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
-    if (fmt == 0) return launch_mma_256_fmt<0>(skip, a, grid, st, ev0, ev1);
-    if (a.qmode == 0) return hipErrorInvalidValue;                   // exact block dots at head dim 256: mma256_kernel
-    if (fmt == 1) return launch_mma_256_fmt<1>(skip, a, grid, st, ev0, ev1);
-    if (fmt == 2) return launch_mma_256_fmt<2>(skip, a, grid, st, ev0, ev1);
+    const bool ex = a.qmode == 0;
+    if (fmt == 0) return launch_mma_256_fmt<0, false>(skip, a, grid, st, ev0, ev1);
+    if (fmt == 1) return ex ? launch_mma_256_fmt<1, true>(skip, a, grid, st, ev0, ev1) : launch_mma_256_fmt<1, false>(skip, a, grid, st, ev0, ev1);
+    if (fmt == 2) return ex ? launch_mma_256_fmt<2, true>(skip, a, grid, st, ev0, ev1) : launch_mma_256_fmt<2, false>(skip, a, grid, st, ev0, ev1);
     return hipErrorInvalidValue;
 }
 

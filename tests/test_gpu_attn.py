@@ -82,19 +82,47 @@ def test_mma256_row_blocks(ws, fmt, rows):
     run_and_check(ws, fmt, 2, rows, 256, 1500, seed=700 + rows + fmt, qmode=bb.QMODE_F16, page_keys=512)
 
 
-@pytest.mark.parametrize("fmt", [bb.FMT_Q8_0, bb.FMT_Q4_0, bb.FMT_F16])
-@pytest.mark.parametrize("rows", [65, 224, 225, 257])
-@pytest.mark.parametrize("workgroups", [0, 1, 400])
-def test_head256_wide_rows(ws, fmt, rows, workgroups):
-    """Head dim 256 above 64 rows with fp16 operands (32-row waves, 256-row blocks): the first row past the 64-row blocks,
-    the last row count with idle waves, the first without, a second row block of one row; over pages that end inside a
-    tile, hold less than one or nothing, in the default chunks, in one chunk per row block (every page change inside the
-    workgroup) and in chunks of one tile."""
-    ws.set_split(mma_workgroups=workgroups)
-    try:
-        run_and_check(ws, fmt, 2, rows, 256, 1037, seed=1700 + rows + fmt, qmode=bb.QMODE_F16, page_keys=[500, 7, 0, 64, 466])
-    finally:
-        ws.set_split()
+@pytest.mark.parametrize("fmt,rows,qmode", [(f, r, bb.QMODE_F16) for f in (bb.FMT_Q8_0, bb.FMT_Q4_0, bb.FMT_F16) for r in (65, 224, 225, 257)]
+                         + [(f, r, bb.QMODE_GGML) for f in (bb.FMT_Q8_0, bb.FMT_Q4_0) for r in (513, 577)])
+def test_head256_wide_rows(ws, fmt, rows, qmode):
+    """Head dim 256 in 32-row waves (256-row blocks; above 64 rows, with the exact block dots above 512, from 384 tiles on):
+    the first rows past the 64-row blocks, the last count with idle waves, the first without, a second or third row block of
+    one row or wave; over pages that end inside a tile, hold less than one or nothing, in the default chunks, in one chunk
+    per row block (every page change inside the workgroup) and in chunks of one or two tiles."""
+    page_keys = [500, 7, 0, 64, 11740]
+    nk, nkv = sum(page_keys), 1
+    print(f"case fmt={fmt} rows={rows} qmode={qmode} nk={nk}", flush=True)
+    K, V, Q, rs = case(fmt, nkv, rows, 256, nk, 1700 + rows + fmt)
+    shape = bb.make_shape(nkv, rows, 256, fmt, qmode, rs=rs)
+    oshape = orc.make_shape(nkv, rows, 256, fmt, orc.QMODE_F16 if qmode == bb.QMODE_F16 else orc.QMODE_GGML, rs=rs)
+    ref = (orc.attn_exact if qmode == bb.QMODE_F16 else orc.attn_ggml)(oshape, Q, K, V, nk)
+    for workgroups in (0, 1, 800):
+        ws.set_split(mma_workgroups=workgroups)
+        try:
+            O, m, l = bb.attn_host(shape, K, V, Q, page_keys=page_keys, ws=ws)
+        finally:
+            ws.set_split()
+        eo, em, el = orc.rel_err(O, m, l, *ref)
+        assert eo < TOL and em < TOL and el < TOL, (workgroups, eo, em, el)
+
+
+@pytest.mark.parametrize("nkv,rows,hd,nk", [(8, 128, 128, 1000), (8, 1000, 128, 2049), (4, 48, 256, 4096), (4, 300, 256, 70), (8, 64, 128, 33)])
+def test_short_context_split(ws, nkv, rows, hd, nk):
+    """Short contexts take fewer chunks than the workgroups that fit (down to one, written directly): the default split
+    against the same call in one chunk and in as many as it has tiles."""
+    K, V, Q, rs = case(bb.FMT_Q8_0, nkv, rows, hd, nk, 2300 + rows)
+    shape = bb.make_shape(nkv, rows, hd, bb.FMT_Q8_0, rs=rs)
+    print(f"case nkv={nkv} rows={rows} hd={hd} nk={nk}", flush=True)
+    outs = []
+    for workgroups in (0, 1, 100000):
+        ws.set_split(mma_workgroups=workgroups)
+        try:
+            outs.append(bb.attn_host(shape, K, V, Q, ws=ws))
+        finally:
+            ws.set_split()
+    for O, m, l in outs[1:]:                                  # the fp16 rounding of P against another reference max
+        eo, em, el = orc.rel_err(O, m, l, *outs[0])
+        assert eo < 1e-3 and em < 1e-6 and el < 1e-3, (eo, em, el)
 
 
 @pytest.mark.parametrize("qmode", [bb.QMODE_GGML, bb.QMODE_F16])
