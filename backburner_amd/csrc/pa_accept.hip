@@ -4,7 +4,8 @@
 // block verification, serve.sh:300-302). Semantics: a_i = argmax_j logits[i][j] with the lowest index on ties (numpy's
 // rule, which also makes the first NaN win); k = the longest prefix with a_i == draft_i (i < n_rows-1); bonus = a_k.
 //
-// Layout: n_rows x splits workgroups; workgroup (row, sp) scans values [S sp, S sp + S) of its row (S = ACCEPT_SEG),
+// Layout: n_rows x splits workgroups; workgroup (row, sp) scans one or more segments of S values of its row (S and their count
+// by the host's rule, accept_split),
 // every thread issuing all its loads at once (S / 1024 16-byte loads, or S / 256 scalar ones when the vocab is not a
 // multiple of 4); its lanes' best values become 64-bit keys (orderable value << 32 | ~index) so that one unsigned max picks the
 // largest value and, among equal values, the lowest index. Each workgroup publishes its key with a write-through store and waits for
@@ -30,14 +31,15 @@ __device__ __forceinline__ unsigned long long accept_key(float x, uint32_t idx) 
 
 __device__ __forceinline__ unsigned long long umax64(unsigned long long a, unsigned long long b) { return a > b ? a : b; }
 
-// The best key of this wave's values of the segment [j0, j1) of row x (64 values per thread: VEC consecutive ones 256 * VEC
-// apart), every load issued at once. The thread's largest value first, then its first place where it is the wave's largest:
+// The best key of this wave's values of the segment [j0, j1) of row x (SEG / 256 values per thread: VEC consecutive ones 256 *
+// VEC apart), every load issued at once. The thread's largest value first, then its first place where it is the wave's largest:
 // about 3.5 vector instructions per value, where a 64-bit key each took fifteen (a workgroup is one wave per SIMD, so nothing
 // hides them). A wave with a NaN anywhere goes over its values again by keys, which rank the first NaN above every value.
-// us per call before and after: [17][151936] 9.05 / 7.5, [33][262144] 18.3 / 12.8, [5][50001] 9.3 / 6.85.
-template <int VEC> __device__ __forceinline__ unsigned long long accept_best(const float * x, int64_t j0, int64_t j1, int t) {
-    constexpr int NU = ACCEPT_SEG / (256 * VEC);
-    const uint32_t n = (uint32_t) (j1 - j0);                         // 1 .. ACCEPT_SEG
+// us per call before and after: [17][151936] 9.05 / 7.5, [33][262144] 18.3 / 12.8, [5][50001] 9.3 / 6.85 (5.0 with the
+// segments by accept_split).
+template <int VEC, int SEG> __device__ __forceinline__ unsigned long long accept_best(const float * x, int64_t j0, int64_t j1, int t) {
+    constexpr int NU = SEG / (256 * VEC);
+    const uint32_t n = (uint32_t) (j1 - j0);                         // 1 .. SEG
     // buffer loads over the segment (values past it read 0 and become -inf in the one segment that has any): no branch per load
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *) (x + j0), (short) 0, (int) (4 * n), 0x00020000);
     float v[NU][VEC];
@@ -51,7 +53,7 @@ template <int VEC> __device__ __forceinline__ unsigned long long accept_best(con
             v[u][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, off, 0, 0));
         }
     }
-    if (n < (uint32_t) ACCEPT_SEG) {
+    if (n < (uint32_t) SEG) {
         #pragma unroll
         for (int u = 0; u < NU; u++)
             #pragma unroll
@@ -91,14 +93,21 @@ template <int VEC> __device__ __forceinline__ unsigned long long accept_best(con
     return best;
 }
 
-__global__ __launch_bounds__(256) void accept_kernel(const AcceptArgs a) {
+// MANY: several segments per workgroup (the loop costs a call of one 0.5 us)
+template <int SEG, bool MANY> __global__ __launch_bounds__(256) void accept_kernel(const AcceptArgs a) {
     __shared__ unsigned long long red[4];
     __shared__ bool last;
     const int row = blockIdx.x / a.splits, sp = blockIdx.x % a.splits;
-    const int64_t j0 = (int64_t) sp * ACCEPT_SEG, j1 = min(a.vocab, j0 + ACCEPT_SEG);
     const float * x = a.logits + (size_t) row * (size_t) a.vocab;
     const int t = threadIdx.x;
-    unsigned long long best = (a.vocab & 3) == 0 ? accept_best<4>(x, j0, j1, t) : accept_best<1>(x, j0, j1, t);
+    auto segment = [&](int64_t j0) {
+        const int64_t j1 = min(a.vocab, j0 + SEG);
+        return (a.vocab & 3) == 0 ? accept_best<4, SEG>(x, j0, j1, t) : accept_best<1, SEG>(x, j0, j1, t);
+    };
+    const int64_t s0 = (int64_t) sp * SEG * (MANY ? a.segs : 1);     // below vocab for every workgroup
+    unsigned long long best = segment(s0);
+    if constexpr (MANY)
+        for (int c = 1; c < a.segs && s0 + (int64_t) c * SEG < a.vocab; c++) best = umax64(best, segment(s0 + (int64_t) c * SEG));
     for (int off = 32; off > 0; off >>= 1) best = umax64(best, __shfl_xor(best, off));
     if ((t & 63) == 0) red[t / 64] = best;
     __syncthreads();
@@ -146,7 +155,12 @@ __global__ __launch_bounds__(256) void accept_kernel(const AcceptArgs a) {
 }
 
 hipError_t launch_accept(const AcceptArgs & a, hipStream_t st) {
-    hipLaunchKernelGGL(accept_kernel, dim3((uint32_t) (a.n_rows * a.splits)), dim3(256), 0, st, a);
+    const dim3 grid((uint32_t) (a.n_rows * a.splits));
+    if (a.seg == 4096 && a.segs == 1) hipLaunchKernelGGL((accept_kernel<4096, false>), grid, dim3(256), 0, st, a);
+    else if (a.seg == 8192 && a.segs == 1) hipLaunchKernelGGL((accept_kernel<8192, false>), grid, dim3(256), 0, st, a);
+    else if (a.seg == 16384 && a.segs == 1) hipLaunchKernelGGL((accept_kernel<16384, false>), grid, dim3(256), 0, st, a);
+    else if (a.seg == 16384) hipLaunchKernelGGL((accept_kernel<16384, true>), grid, dim3(256), 0, st, a);
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 

@@ -75,14 +75,6 @@ hipError_t launch_normalise(int hd, const float * O, const float * m, const floa
 hipError_t launch_coattn(int hd, const uint16_t * Oh, const float * lse, const float * Oloc, const float * mloc,
                          const float * lloc, uint64_t rows, float * out, float * lse_out, hipStream_t st);
 
-#ifndef PA_ACCEPT_SEG
-#define PA_ACCEPT_SEG 16384
-#endif
-// logits per acceptance workgroup (a multiple of 1024): fewer, fuller workgroups, and fewer keys for the last one to fold.
-// [17][151936] fp32, kernel time with a 64-bit key per value: 7.2 us at 16384 (170 workgroups), 8.3 at 8192, 8.8 at 32768,
-// 12.0 at 4096
-constexpr int ACCEPT_SEG = PA_ACCEPT_SEG;
-
 struct AcceptArgs {
     const float * logits;
     const int32_t * draft;
@@ -90,7 +82,8 @@ struct AcceptArgs {
     unsigned long long * part;      // [n_rows][splits] packed (orderable value, ~index)
     unsigned int * counter;         // one counter, zero between calls (the last block resets it)
     int64_t vocab;
-    int n_rows, splits;
+    int n_rows, splits;             // workgroups per row, each `segs` consecutive segments of `seg` values (4096, 8192, 16384)
+    int seg, segs;
 };
 hipError_t launch_accept(const AcceptArgs & a, hipStream_t st);
 

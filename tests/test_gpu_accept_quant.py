@@ -91,6 +91,18 @@ def test_accept_segment_edges(ws, vocab):
     assert np.array_equal(am, np.argmax(logits, axis=1))
 
 
+def test_accept_several_segments_per_workgroup(ws):
+    """64 rows of 13 segments: 832 workgroups of one segment become 256 of four, the last one shorter."""
+    vocab, n = 12 * 16384 + 5, 64
+    rng = np.random.default_rng(77)
+    logits = rng.standard_normal((n, vocab)).astype(np.float32)
+    at = rng.integers(0, vocab, n); at[:4] = [0, vocab - 1, 4 * 16384 - 1, 4 * 16384]
+    logits[np.arange(n), at] = 50.0
+    logits[5, at[5]:] = np.nan
+    am = gpu_accept(ws, logits, np.zeros(n - 1, np.int32))[2]
+    assert np.array_equal(am, np.argmax(logits, axis=1))
+
+
 def test_accept_repeated_calls_reset_counter(ws):
     rng = np.random.default_rng(9)
     for it in range(5):
