@@ -682,11 +682,11 @@ bool pages_aligned(const char * fn, void * const * kp, void * const * vp, uint32
     return true;
 }
 
-// the launches of a converting APPEND: rows of up to APPEND_SEGS pages each, and at most 2^23 workgroups (2^31 threads);
+// the launches of a converting APPEND: rows of up to APPEND_SEGS pages each, at most 65,535 (a grid dimension) and 2^23 workgroups;
 // `row` = bytes of a source row, the rest of `a` filled in
 int append_launches(AppendArgs & a, bool from_f32, void * const * kp, void * const * vp, uint32_t page_keys, uint32_t pos0,
                     const uint8_t * K, const uint8_t * V, size_t row, uint32_t n, hipStream_t st) {
-    const uint64_t max_rows = std::max<uint64_t>(1, (1u << 23) / ((2ull * a.nkv * (a.hd / 32) + 15) / 16));
+    const uint64_t max_rows = std::min<uint64_t>(65535, std::max<uint64_t>(1, (1u << 23) / ((2ull * a.nkv * (a.hd / 32) + 15) / 16)));
     for (uint32_t done = 0; done < n;) {
         const uint32_t pi = (pos0 + done) / page_keys, off = (pos0 + done) % page_keys;
         const uint32_t take = (uint32_t) std::min<uint64_t>({n - done, max_rows, (uint64_t) APPEND_SEGS * page_keys - off});

@@ -98,15 +98,15 @@ struct AppendAt {                   // this lane's block: its values (row j, hea
 };
 __device__ __forceinline__ AppendAt append_at(const AppendArgs & a) {
     AppendAt r;
-    const uint32_t nb = a.hd / 32, lnb = nb == 4 ? 2u : 3u, per_t = a.nkv * nb, wpr = (2 * per_t + 15) / 16;
-    const uint32_t j = blockIdx.x / wpr, q = (blockIdx.x % wpr) * 16 + threadIdx.x / 16;
+    const uint32_t nb = a.hd / 32, lnb = nb == 4 ? 2u : 3u, per_t = a.nkv * nb;
+    const uint32_t j = blockIdx.y, q = blockIdx.x * 16 + threadIdx.x / 16;
     r.live = q < 2 * per_t;                                          // whole 16-lane rows leave together
     r.tensor = q >= per_t ? 1u : 0u;
     const uint32_t u = q - r.tensor * per_t;
     r.j = j;
     r.h = u >> lnb;
     r.b = u & (nb - 1);
-    const uint32_t p = a.off0 + j, pg = p / a.page_keys;             // off0 < page_keys: the first segment's offset
+    const uint32_t p = a.off0 + j, pg = p < a.page_keys ? 0u : p / a.page_keys;   // off0 < page_keys: the first segment's offset
     r.row = (r.tensor ? a.vdst[pg] : a.kdst[pg]) + (size_t) (p - pg * a.page_keys) * a.rs;
     return r;
 }
@@ -144,7 +144,7 @@ hipError_t launch_quantize(int fmt, const float * x, void * y, int64_t n, hipStr
 hipError_t launch_append(bool from_f32, const AppendArgs & a, hipStream_t st) {
     const uint32_t wpr = (2 * a.nkv * (a.hd / 32) + 15) / 16;        // workgroups per row
     if (a.n == 0) return hipSuccess;
-    const dim3 grid(a.n * wpr);
+    const dim3 grid(wpr, a.n);                                       // n <= 65,535 (the host's launches)
     if (from_f32) hipLaunchKernelGGL(append_quant_kernel, grid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL(append_f16_kernel, grid, dim3(256), 0, st, a);
     return hipGetLastError();
