@@ -555,15 +555,17 @@ extern "C" int pa_hip_attn(pa_hip_ws * ws, const pa_hip_shape * s, const void * 
 
 namespace {
 // The acceptance's segments. Smaller ones end sooner, but every workgroup counts itself done on one address (about 20 ns each),
-// so the smallest that keeps to 140 workgroups is taken, and above 768 of the largest a workgroup takes several, 256 in all.
+// so the smallest that keeps to 140 workgroups is taken, and above 768 (ACCEPT_MAX_WG) of the largest a workgroup takes several,
+// 256 in all.
 // us per call at 4096 / 8192 / 16384 values: [2][32000] 4.4 / 4.9 / 6.0, [5][50001] 4.9 / 5.3 / 6.8, [5][128256] 5.9 / 5.4 /
 // 6.6, [33][32000] 8.3 / 6.9 / 7.7, [17][128256] 11.2 / 8.1 / 7.1, [17][151936] 12.3 / 8.7 / 7.5; with one / several segments
 // per workgroup: [64][262144] 24.7 / 20.0, [33][262144] 12.8 / 12.1 (the loop in every call), [33][151936] 9.9 / 10.5.
+constexpr int ACCEPT_MAX_WG = 768;
 void accept_split(int n_rows, int64_t vocab, int & seg, int & segs, int & splits) {
     auto count = [&](int64_t span) { return (int) ((vocab + span - 1) / span); };
     segs = 1;
     for (seg = 4096; seg < 16384 && (int64_t) n_rows * count(seg) > 140; seg *= 2) {}
-    if ((int64_t) n_rows * count(seg) > 768)
+    if ((int64_t) n_rows * count(seg) > ACCEPT_MAX_WG)
         while ((int64_t) n_rows * count((int64_t) seg * segs) > 256 && segs < count(seg)) segs++;
     splits = count((int64_t) seg * segs);
 }
@@ -577,8 +579,9 @@ extern "C" int pa_hip_accept(pa_hip_ws * ws, const float * logits, int n_rows, i
     if ((vocab & 3) == 0 && ((uintptr_t) logits & 15)) { set_err("pa_hip_accept: logits must be 16-byte aligned"); return -1; }
     AcceptArgs a;
     accept_split(n_rows, vocab, a.seg, a.segs, a.splits);
-    // (room for any small call, so that one over more rows or segments does not have to grow it)
-    const size_t need = std::max<size_t>((size_t) n_rows * a.splits, 256) * sizeof(unsigned long long);
+    // Room for every shape from the first call on: the count does not grow with the shape (64 rows of 262,144 values take 256
+    // workgroups, 48 rows 768), and a captured call must not find the workspace of a larger eager one too small.
+    const size_t need = (size_t) ACCEPT_MAX_WG * sizeof(unsigned long long);
     if (!ensure(ws, ws->apart, ws->apart_cap, need, (hipStream_t) stream, true, "hipMalloc accept partials")) return -1;
     a.logits = logits; a.draft = draft; a.out = out; a.part = ws->apart; a.counter = ws->acount;
     a.vocab = vocab; a.n_rows = n_rows;

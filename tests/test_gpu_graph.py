@@ -109,3 +109,52 @@ def test_graph_replays_accept():
         if gx:
             syn.pa_synth_graph_free(gx)
         ws.close()
+
+
+def captured_replays(syn, ws, call, dout, stream, compare):
+    """call(ws) captured on `stream` (no eager call of it before) and replayed over poisoned output, compare(bytes) each."""
+    n = dout.nbytes
+    assert syn.pa_synth_capture_begin(stream) == 0
+    refused, gx = None, None
+    try:
+        call(ws)
+    except bb.PaHipError as e:
+        refused = str(e)
+    gx = syn.pa_synth_capture_end(stream)
+    try:
+        assert refused is None, refused
+        assert gx, "capture failed"
+        for _ in range(3):
+            dout.upload(np.full(n, 0x7f, np.uint8))
+            assert syn.pa_synth_graph_launch(gx, stream) == 0
+            assert syn.pa_synth_stream_sync(stream) == 0
+            compare(dout.download(np.uint8))
+    finally:
+        if gx:
+            syn.pa_synth_graph_free(gx)
+
+
+@pytest.mark.parametrize("rows", [33, 48])
+def test_accept_captured_after_a_larger_eager_call(rows):
+    """One eager call of the largest shape sizes the workspace for every smaller one: 64 rows of 262,144 values take several
+    segments per workgroup (256 partials), 33 and 48 rows one each (528 and 768)."""
+    print(f"graph accept {rows} rows after 64", flush=True)
+    syn = bb.synth()
+    rng = np.random.default_rng(45)
+    logits = rng.standard_normal((64, 262144), dtype=np.float32)
+    draft = rng.integers(0, 262144, 63).astype(np.int32)
+    for i in range(6):
+        logits[i, draft[i]] = 50.0
+    dl, dd = bb.DeviceBuffer.from_array(logits), bb.DeviceBuffer.from_array(draft)
+    big, do = bb.DeviceBuffer(66 * 4), bb.DeviceBuffer((2 + rows) * 4)
+    k, bonus, am = orc.accept(logits[:rows], draft[:rows - 1])
+    want = np.concatenate([[k, bonus], am]).astype(np.int32)
+    ws = bb.Workspace()
+    stream = syn.pa_synth_stream_new()
+    try:
+        ws.accept(dl.ptr, 64, 262144, dd.ptr, big.ptr, stream)
+        assert syn.pa_synth_stream_sync(stream) == 0
+        captured_replays(syn, ws, lambda w: w.accept(dl.ptr, rows, 262144, dd.ptr, do.ptr, stream), do, stream,
+                         lambda got: np.testing.assert_array_equal(got.view(np.int32), want))
+    finally:
+        ws.close()
