@@ -96,6 +96,13 @@ struct pa_hip_ws {
 
 namespace {
 
+bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    const bool on = hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+    if (!on) (void) hipGetLastError();
+    return on;
+}
+
 // A device buffer of the workspace with room for need_bytes. A larger one replaces it when needed: keep_old retires the
 // old one (freed with the workspace: the engine path's buffers, which a captured graph may hold), otherwise it is freed
 // once the stream is idle (the synchronous sme_* staging). Growth while `st` is being captured is refused: hipMalloc
@@ -103,13 +110,11 @@ namespace {
 template <typename T>
 bool ensure(pa_hip_ws * ws, T *& p, size_t & cap, size_t need_bytes, hipStream_t st, bool keep_old, const char * what) {
     if (need_bytes <= cap && p) return true;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) {
+    if (capturing(st)) {
         set_err(std::string(what) + ": the workspace must grow (" + std::to_string(need_bytes) +
                 " bytes) inside a stream capture; make one eager call of the largest shape before capturing");
         return false;
     }
-    (void) hipGetLastError();
     const size_t sz = std::max<size_t>({need_bytes, 2 * cap, 256});
     T * np = nullptr;
     if (!hip_ok(hipMalloc((void **) &np, sz), what)) return false;
@@ -235,6 +240,15 @@ struct Call {
         po = ws->po;
         pml = ws->pml;
         return true;
+    }
+    bool fits(uint64_t rows, uint32_t hd) const {   // without growing the workspace
+        return rows * hd * sizeof(float) <= ws->po_cap && rows * sizeof(float2) <= ws->pml_cap;
+    }
+    // Room in the workspace beyond the call's own slots, for later calls. Taken where it can be had, never a reason to refuse
+    // the call: nothing is asked for inside a capture, and a failed allocation is forgotten.
+    void reserve(uint64_t rows, uint32_t hd, hipStream_t st) {
+        if (fits(rows, hd) || capturing(st)) return;
+        if (!slots(rows, hd, st)) (void) hipGetLastError();
     }
     // the merge of the call's slots: the reply format when asked for, else (O, m, l)
     bool merge(MergeArgs & ma, int hd, hipStream_t st) {
@@ -410,22 +424,21 @@ int attn_mma(Call & cx, const pa_hip_shape * s, const void * const * k_pages, co
         for_launches(nkeys, n_pages, [&](int, int, uint64_t tiles, uint64_t) { n_slots += chunking(tiles, cap, tpc); });
     }
     const bool direct = n_launch == 1 && n_slots == 1;
-    // a workspace gets room for one round of workgroups of either kernel whatever this context pays for, so that a call over
-    // more keys does not have to grow it (which a stream capture refuses)
-    uint64_t room = direct ? 0 : n_slots * rows_per_slot;
+    // a workspace gets the room that one round of workgroups of either kernel would take over this context, whatever the
+    // context pays for, so that calls of other shapes find what they need there when they are captured
     if (!cx.fixed && cx.mma_workgroups == 0 && cx.chunk_keys == 0) {
         auto round_rows = [&](uint32_t block, uint64_t workgroups, uint64_t tiles) {
             const uint64_t n = std::max<uint64_t>(1, workgroups / ((uint64_t) s->nkv * ((s->rows + block - 1) / block)));
             return std::min(n, tiles) * rows_per_slot;
         };
-        uint64_t rows = 0;
+        uint64_t room = 0;
         for_launches(nkeys, n_pages, [&](int, int, uint64_t tiles, uint64_t) {
-            rows += s->hd == 256 ? std::max(round_rows(64, 512, tiles), s->rows > 64 ? round_rows(256, 256, tiles) : 0)
+            room += s->hd == 256 ? std::max(round_rows(64, 512, tiles), s->rows > 64 ? round_rows(256, 256, tiles) : 0)
                                  : round_rows(rpw * nw, 2048 / nw, tiles);
         });
-        if (rows > rows_per_slot) room = std::max(room, rows);
+        if (room > rows_per_slot) cx.reserve(room, s->hd, st);
     }
-    if (room > 0 && !cx.slots(room, s->hd, st)) return -1;
+    if (!direct && !cx.slots(n_slots * rows_per_slot, s->hd, st)) return -1;
     uint32_t li = 0, slot0 = 0;
     bool ok = true;
     for_launches(nkeys, n_pages, [&](int p0, int np, uint64_t tiles, uint64_t) {

@@ -158,3 +158,66 @@ def test_accept_captured_after_a_larger_eager_call(rows):
                          lambda got: np.testing.assert_array_equal(got.view(np.int32), want))
     finally:
         ws.close()
+
+
+def attn_problem(fmt, nkv, rows, hd, nk, qmode, seed):
+    """shape, pages and Q of one call, and a run(ws, out, stream) of it."""
+    hb = orc.head_bytes(fmt, hd); rs = nkv * hb
+    rng = np.random.default_rng(seed)
+    K = orc.fill_rows(seed, fmt, nkv, hd, nk, rs=rs); V = orc.fill_rows(seed + 1, fmt, nkv, hd, nk, rs=rs)
+    n = nkv * rows
+    dq = bb.DeviceBuffer.from_array(rng.standard_normal((n, hd), dtype=np.float32))
+    shape, pages = bb.make_shape(nkv, rows, hd, fmt, qmode, rs=rs), bb.pages_from_rows(K, V, rs, 4096)
+
+    def run(ws, out, st):
+        ws.attn(shape, pages, dq.ptr, out.ptr, out.ptr + n * hd * 4, out.ptr + n * hd * 4 + n * 4, st)
+
+    def split(got):
+        f = got.view(np.float32)
+        return f[:n * hd].reshape(n, hd), f[n * hd:n * hd + n], f[n * hd + n:]
+
+    return run, split, n * hd * 4 + n * 8, pages
+
+
+def check_captured_after(first, then):
+    """`then` captured on a workspace that has seen the eager call `first` (None: a fresh one): accepted, and every replay
+    equal to the eager result on another workspace up to the fp16 rounding of P against another chunk's reference max."""
+    print(f"capture {then} after {first}", flush=True)
+    syn = bb.synth()
+    ws, ws2 = bb.Workspace(), bb.Workspace()
+    stream = syn.pa_synth_stream_new()
+    held = []
+    try:
+        if first:
+            run, _, nbytes, pages = attn_problem(*first, seed=600)
+            held.append(pages)
+            run(ws, bb.DeviceBuffer(nbytes), stream)
+            assert syn.pa_synth_stream_sync(stream) == 0
+        run, split, nbytes, pages = attn_problem(*then, seed=700)
+        held.append(pages)
+        dout, dref = bb.DeviceBuffer(nbytes), bb.DeviceBuffer(nbytes)
+        run(ws2, dref, stream)
+        assert syn.pa_synth_stream_sync(stream) == 0
+        ref = split(dref.download(np.uint8))
+
+        def compare(got):
+            eo, em, el = orc.rel_err(*split(got), *ref)
+            assert eo < 1e-3 and em < 1e-6 and el < 1e-3, (eo, em, el)
+
+        captured_replays(syn, ws, lambda w: run(w, dout, stream), dout, stream, compare)
+    finally:
+        ws.close()
+        ws2.close()
+        for p in held:
+            p.close()
+
+
+@pytest.mark.parametrize("first,then", [
+    # 10 chunks of 768 padded rows per head, then 50 of 128 that a whole round would make 64
+    ((bb.FMT_Q8_0, 8, 520, 128, 6400, bb.QMODE_GGML), (bb.FMT_Q8_0, 8, 48, 128, 6400, bb.QMODE_GGML)),
+    # one chunk, written directly, needs no slots (a longer context would)
+    (None, (bb.FMT_Q8_0, 8, 4096, 256, 64, bb.QMODE_F16)),
+])
+def test_captured_call_needs_no_headroom(first, then):
+    """The room that a workspace takes ahead for longer contexts is no reason to refuse a captured call whose own slots fit."""
+    check_captured_after(first, then)
