@@ -423,6 +423,15 @@ int attn_mma(Call & cx, const pa_hip_shape * s, const void * const * k_pages, co
         n_slots = 0;
         for_launches(nkeys, n_pages, [&](int, int, uint64_t tiles, uint64_t) { n_slots += chunking(tiles, cap, tpc); });
     }
+    // A captured call cannot grow the workspace. mma_kernel's 256-row blocks at head dim 256 take more chunks than 64-row blocks
+    // do, whose count a workspace that has run shorter contexts or fewer rows holds: the call then takes no more than that.
+    const bool by_keys = cx.chunk_keys > 0 && cx.mma_workgroups == 0;
+    if (!cx.fixed && s->hd == 256 && !h256 && !by_keys && !(n_launch == 1 && n_slots == 1) &&
+        !cx.fits(n_slots * rows_per_slot, s->hd) && capturing(st)) {
+        cap = std::max<uint64_t>(1, (cx.mma_workgroups > 0 ? (uint64_t) cx.mma_workgroups : 512u) / ((uint64_t) s->nkv * (qr / 64)));
+        n_slots = 0;
+        for_launches(nkeys, n_pages, [&](int, int, uint64_t tiles, uint64_t) { n_slots += chunking(tiles, cap, tpc); });
+    }
     const bool direct = n_launch == 1 && n_slots == 1;
     // a workspace gets the room that one round of workgroups of either kernel would take over this context, whatever the
     // context pays for, so that calls of other shapes find what they need there when they are captured

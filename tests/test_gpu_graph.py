@@ -221,3 +221,16 @@ def check_captured_after(first, then):
 def test_captured_call_needs_no_headroom(first, then):
     """The room that a workspace takes ahead for longer contexts is no reason to refuse a captured call whose own slots fit."""
     check_captured_after(first, then)
+
+
+@pytest.mark.parametrize("first,then", [
+    # 128 chunks of 64 rows per head, then 32 of 256 in 64-row blocks where 256-row blocks would take 64
+    ((bb.FMT_Q8_0, 4, 48, 256, 16384, bb.QMODE_F16), (bb.FMT_F16, 4, 240, 256, 33333, bb.QMODE_F16)),
+    ((bb.FMT_Q8_0, 4, 48, 256, 16384, bb.QMODE_F16), (bb.FMT_Q8_0, 4, 600, 256, 20000, bb.QMODE_GGML)),
+    # one chunk of 64-row blocks, two of 256-row blocks
+    (None, (bb.FMT_Q4_0, 2, 16384, 256, 12288, bb.QMODE_F16)),
+])
+def test_captured_head256_call_in_the_slots_of_64_row_blocks(first, then):
+    """Head dim 256 over long contexts: the 256-row blocks take more chunks than the 64-row blocks that short contexts run; a
+    captured call whose workspace holds the latter's count takes that."""
+    check_captured_after(first, then)
