@@ -198,9 +198,14 @@ namespace {
 // round and are slower). q4_0, twice the work per byte: four per CU (45.4-46.4 against 49.5-50.2 us at three).
 constexpr int DEC_TARGET_WG_Q8 = 768, DEC_TARGET_WG_Q4 = 1024;
 
-// The split of the matrix-core kernels (attn_mma): what a step of one tile costs (head dim 128, head dim 256, and there with
-// the exact block dots), the rate at which slots are written and read back, and the merge's launch
-constexpr double TILE_US_128 = 1.5, TILE_US_256 = 2.4, TILE_US_256_EX = 3.0, SLOT_BYTES_PER_US = 4.5e6, MERGE_US = 4.0;
+// The split of the matrix-core kernels (attn_mma): what a step of one tile costs with one workgroup on a CU (TWO_PER_CU times it
+// with two), what a tile of a call's only chunk costs, and the gain below which a call keeps a whole round of workgroups; the
+// slots' time, written and read back; and what a merge costs, with its share per MB of result. Fitted to 3,600 shapes of 12 to
+// 4,000 rows, 1 to 32 heads and 64 to 33,333 keys.
+struct MmaTile { double step, only, gain; };
+constexpr MmaTile TILE_128_W4 = {0.8, 1.25, 0}, TILE_128_W4_EX = {1.1, 1.7, 0}, TILE_128_W8 = {1.5, 1.4, 0}, TILE_128_W8_EX = {1.8, 1.8, 0};
+constexpr MmaTile TILE_256 = {1.2, 1.75, 1}, TILE_256_EX = {1.7, 2.4, 1}, TILE_256_WIDE = {2.4, 1.75, 0}, TILE_256_WIDE_EX = {3.0, 2.4, 0};
+constexpr double TWO_PER_CU = 1.3, SLOT_US_PER_MB = 0.444, MERGE_US = 4.6, MERGE_US_PER_MB = 2.8;
 
 // One call of the engine path: where its split-K slots go, its geometry overrides, its timing events and, for
 // pa_hip_attn_reply, the reply target the merge writes instead of (O, m, l).
@@ -390,20 +395,31 @@ int attn_mma(Call & cx, const pa_hip_shape * s, const void * const * k_pages, co
     // key chunks: by default one round of resident workgroups (one of 8 waves or two of 4 per CU, 256 CUs); a second,
     // partial round costs more than the extra slots save
     const uint64_t target = cx.mma_workgroups > 0 ? (uint64_t) cx.mma_workgroups : 256u * 8 / nw;
-    // fewer chunks where a short context does not pay for them: n chunks take tiles / n steps, and their slots are written
-    // and read again, so the cost is least at n = the root of tiles x tile time / slot time; one chunk, written directly, where
-    // that costs no more than the merge's launch on top. us per call with one round of workgroups whatever the context and
-    // so: 8 heads x 128 rows at head dim 128 over 1,000 f16 keys 19.5 / 14.3, over 4,096 25.7 / 20.0; 4,000 rows over 300 q8_0
-    // keys 34.6 / 25.5, over 1,000 48.9 / 45.0; 4 heads x 48 rows at head dim 256 over 4,096 q8_0 keys 25.8 / 18.6, 300 rows
-    // over 1,000 27.1 / 20.8; from 16,384 keys on the count is one round's again.
+    // Fewer chunks where a short context does not pay for them. One chunk, written directly, takes every tile in turn and saves
+    // the slots and the merge: us with one / several, 8 heads x 129 rows in exact block dots over 64 q8_0 keys 11.9 / 13.1, over
+    // 128 keys 14.4 / 13.8; 2,000 rows over 320 keys 24.1 / 27.2. n chunks take tiles / n steps, and their slots are written
+    // and read again, so the cost is least at n = the root of tiles x slot time / step. Of the 4-wave workgroups a round holds
+    // two per CU: between one and two, the CUs that hold two set the time while the chunks are longer than a whole round's, so
+    // it is one at most, or the round: us with 64 / 43 / 32 chunks, 8 heads x 96 rows over 8,192 q8_0 keys 24.0 / 25.4 / 21.9;
+    // with 32 / 22 / 16, head dim 256, 4 heads x 256 rows over 4,096 keys 32.2 / 33.5 / 26.7.
     auto pays = [&](uint64_t tiles) -> uint64_t {
-        const double tile_us = s->hd == 128 ? TILE_US_128 : ex ? TILE_US_256_EX : TILE_US_256;
-        const double slot_us = 2.0 * s->nkv * s->rows * (s->hd * sizeof(float) + sizeof(float2)) / SLOT_BYTES_PER_US;
-        // tiles per chunk: the better of the two counts around the root
-        auto cost = [&](uint64_t t) { return t * tile_us + (tiles + t - 1) / t * slot_us; };
-        uint64_t t = std::max<uint64_t>(1, (uint64_t) std::sqrt(tiles * slot_us / tile_us));
-        if (cost(t + 1) < cost(t)) t++;
-        return tiles * tile_us <= cost(t) + MERGE_US ? 1 : (tiles + t - 1) / t;
+        const MmaTile & tile = s->hd == 128 ? (nw == 4 ? (ex ? TILE_128_W4_EX : TILE_128_W4) : ex ? TILE_128_W8_EX : TILE_128_W8)
+                             : h256 ? (ex ? TILE_256_EX : TILE_256) : ex ? TILE_256_WIDE_EX : TILE_256_WIDE;
+        const double slot_mb = (double) s->nkv * s->rows * (s->hd * sizeof(float) + sizeof(float2)) * 1e-6;
+        if (tiles * tile.only <= MERGE_US + MERGE_US_PER_MB * slot_mb) return 1;
+        const double slot_us = SLOT_US_PER_MB * slot_mb;
+        // tiles per chunk: the better of the two counts around the root, at most one workgroup per CU
+        const uint64_t round = std::max<uint64_t>(1, target / units), single = std::max<uint64_t>(1, 256 / units);
+        auto cost = [&](uint64_t t, double step) { return t * step + (tiles + t - 1) / t * slot_us; };
+        uint64_t t = std::max<uint64_t>(1, (uint64_t) std::sqrt(tiles * slot_us / tile.step));
+        if (cost(t + 1, tile.step) < cost(t, tile.step)) t++;
+        t = std::max(t, (tiles + single - 1) / single);
+        if (nw == 4) {
+            const uint64_t tr = (tiles + round - 1) / round;
+            const double step = (tiles + tr - 1) / tr * units > 256 ? TWO_PER_CU * tile.step : tile.step;
+            if (cost(tr, step) < cost(t, tile.step) + tile.gain) return round;
+        }
+        return (tiles + t - 1) / t;
     };
     auto chunking = [&](uint64_t tiles, uint64_t cap, uint32_t & tpc) {
         uint64_t want = std::max<uint64_t>(1, std::min(target / units, cap));
