@@ -198,13 +198,14 @@ namespace {
 // round and are slower). q4_0, twice the work per byte: four per CU (45.4-46.4 against 49.5-50.2 us at three).
 constexpr int DEC_TARGET_WG_Q8 = 768, DEC_TARGET_WG_Q4 = 1024;
 
-// The split of the matrix-core kernels (attn_mma): what a step of one tile costs with one workgroup on a CU (TWO_PER_CU times it
-// with two), what a tile of a call's only chunk costs, and the gain below which a call keeps a whole round of workgroups; the
-// slots' time, written and read back; and what a merge costs, with its share per MB of result. Fitted to 3,600 shapes of 12 to
-// 4,000 rows, 1 to 32 heads and 64 to 33,333 keys.
-struct MmaTile { double step, only, gain; };
-constexpr MmaTile TILE_128_W4 = {0.8, 1.25, 0}, TILE_128_W4_EX = {1.1, 1.7, 0}, TILE_128_W8 = {1.5, 1.4, 0}, TILE_128_W8_EX = {1.8, 1.8, 0};
-constexpr MmaTile TILE_256 = {1.2, 1.75, 1}, TILE_256_EX = {1.7, 2.4, 1}, TILE_256_WIDE = {2.4, 1.75, 0}, TILE_256_WIDE_EX = {3.0, 2.4, 0};
+// The split of the matrix-core kernels (mma_chunks): what a step of one tile costs with one workgroup on a CU (TWO_PER_CU times it
+// with two), what a tile of a call's only chunk costs, the gain below which 4-wave calls keep the larger count, and the longest
+// chunk, in tiles, with which they take one workgroup per CU; the slots' time, written and read back; and what a merge costs,
+// with its share per MB of result. Fitted to 3,600 shapes of 12 to 4,000 rows, 1 to 32 heads and 64 to 33,333 keys.
+struct MmaTile { double step, only, gain; uint32_t alone; };
+constexpr MmaTile TILE_128_W4 = {0.8, 1.25, 0, 10}, TILE_128_W4_EX = {1.1, 1.7, 0, 10}, TILE_128_W8 = {1.5, 1.4}, TILE_128_W8_EX = {1.5, 1.8};
+constexpr MmaTile TILE_256 = {1.2, 1.75, 1, 12}, TILE_256_EX = {1.7, 2.4, 1, 10}, TILE_256_WIDE = {1.4, 1.75},
+                  TILE_256_WIDE_SKIP = {2.4, 1.75}, TILE_256_WIDE_EX = {2.6, 2.4};
 constexpr double TWO_PER_CU = 1.3, SLOT_US_PER_MB = 0.444, MERGE_US = 4.6, MERGE_US_PER_MB = 2.8;
 
 // One call of the engine path: where its split-K slots go, its geometry overrides, its timing events and, for
@@ -363,67 +364,128 @@ int attn_decode(Call & cx, const pa_hip_shape * s, const void * const * k_pages,
     return cx.merge(ma, (int) s->hd, st) ? 0 : -1;
 }
 
+// A matrix-core call's kernel and geometry. mma_kernel: 32 rows per wave, 8 waves above 128 rows (prefill) and at head dim 256, 4
+// otherwise (verify, short verify blocks, f16 decode). mma256_kernel (h256): 16 rows per wave, 4 waves (the reference's 48 rows
+// per KV head fill three).
+struct MmaForm {
+    bool h256, ex;                    // ex: exact block dots (ggml's rounding over quantized K)
+    uint32_t nw, rpw, nrb, units;     // waves, rows per wave, row blocks per KV head, workgroups per chunk
+    double slot_mb;                   // one chunk's slots
+    MmaTile tile;
+};
+
+MmaForm mma_form(const pa_hip_shape * s, bool wide) {
+    MmaForm f;
+    f.ex = s->qmode == PA_QMODE_GGML && s->fmt != PA_FMT_F16;
+    f.h256 = s->hd == 256 && !wide;
+    f.nw = f.h256 ? 4u : s->rows > 128 || s->hd == 256 ? 8u : 4u;
+    f.rpw = f.h256 ? 16u : 32u;
+    f.nrb = (s->rows + f.rpw * f.nw - 1) / (f.rpw * f.nw);
+    f.units = s->nkv * f.nrb;
+    f.slot_mb = (double) s->nkv * s->rows * (s->hd * sizeof(float) + sizeof(float2)) * 1e-6;
+    f.tile = s->hd == 128 ? (f.nw == 4 ? (f.ex ? TILE_128_W4_EX : TILE_128_W4) : f.ex ? TILE_128_W8_EX : TILE_128_W8)
+           : f.h256 ? (f.ex ? TILE_256_EX : TILE_256) : f.ex ? TILE_256_WIDE_EX : s->rows <= 224 ? TILE_256_WIDE_SKIP : TILE_256_WIDE;
+    return f;
+}
+
+// The default chunk count of a launch: at most one round of resident workgroups (one of 8 waves or two of 4 per CU, 256 CUs; a
+// second, partial round costs more than the extra slots save), fewer where a short context does not pay for them.
+// One chunk, written directly, takes every tile in turn and saves the slots and the merge: us with one / several, 8 heads x 129
+// rows in exact block dots over 64 q8_0 keys 11.9 / 13.1, over 128 keys 14.4 / 13.8; 2,000 rows over 320 keys 24.1 / 27.2. n
+// chunks take tiles / n steps, and their slots are written and read again, so the cost is least at n = the root of tiles x slot
+// time / step. Of the 4-wave workgroups a round holds two per CU. One per CU is 15-25 % faster as long as its chunks are short:
+// over 1,600 shapes the time against the whole round is 0.77 at 2 tiles, 0.85 at 6, 0.9 at 10 (at most 1.05), 0.95-1.06 at 16,
+// 1.0-1.1 at 24; few rows leave less to save in slots, so the cost is compared as well. Between one and two the CUs that hold
+// two set the time while the chunks are longer than a whole round's, so it is never taken: us with 64 / 43 / 32 chunks, 8 heads
+// x 96 rows over 8,192 q8_0 keys 24.0 / 25.4 / 21.9; with 32 / 22 / 16, head dim 256, 4 heads x 256 rows over 4,096 keys 32.2 /
+// 33.5 / 26.7.
+uint64_t mma_chunks(const MmaForm & f, uint64_t tiles) {
+    if (tiles * f.tile.only <= MERGE_US + MERGE_US_PER_MB * f.slot_mb) return 1;
+    const uint64_t round = std::max<uint64_t>(1, 2048u / f.nw / f.units), single = std::max<uint64_t>(1, 256 / f.units);
+    const double slot_us = SLOT_US_PER_MB * f.slot_mb;
+    const uint64_t t1 = (tiles + single - 1) / single;               // tiles per chunk with one workgroup per CU
+    // tiles per chunk: the better of the two counts around the root
+    auto cost = [&](uint64_t t) { return t * f.tile.step + (tiles + t - 1) / t * slot_us; };
+    uint64_t t = std::max<uint64_t>(1, (uint64_t) std::sqrt(tiles * slot_us / f.tile.step));
+    if (cost(t + 1) < cost(t)) t++;
+    t = std::max(t, t1);
+    if (f.nw == 4) {
+        if (cost(t1) < cost(t) + f.tile.gain) t = t1;
+        const uint64_t tr = (tiles + round - 1) / round, n = (tiles + tr - 1) / tr;
+        if (n * f.units > 256 && (t1 > f.tile.alone || tr * TWO_PER_CU * f.tile.step + n * slot_us < cost(t))) return n;
+    }
+    return (tiles + t - 1) / t;
+}
+
+// Head dim 256 in mma_kernel (256-row blocks) instead of mma256_kernel (64-row blocks)? Each 16-row wave of the latter reads a
+// whole tile from LDS for half the rows and each 64-row block dequantizes it again; but an 8-wave workgroup starts and ends about
+// 10 us later, so only contexts of at least 384 tiles (fewer above 512 rows) and, in the exact block dots, whose 32-row form
+// converts and scales each dot in vector instructions, only more than 512 rows are asked about. There the time of both is
+// estimated: 256-row blocks take fewer steps where they are full, but up to twice the slots, which cost most past the 32 MB
+// that the L2s hold. The estimate (fitted to 750 such calls, 2 to 5 % off; the choice 0.1 % off the better one on average) is a
+// start, a time per step, a time per MB of slots and the wider merge of more than 64 slots.
+// us per call, mma256_kernel / mma_kernel, 4 heads, fp16 operands, 16,384 q8_0 keys: 72 rows 33.3 / 26.7, 256 rows 50.5 / 59.7,
+// 300 rows 57.6 / 56.3, 512 rows 77.1 / 81.6, 1,024 rows 130 / 108; f16 keys, 256 rows 46.9 / 58.6, 33,333 of them 70.9 / 74;
+// exact block dots, 12,288 q8_0 keys: 513 rows 90 / 94, 900 rows 132 / 111.
+struct Mma256Time {
+    double start, step, mb;           // mma256_kernel
+    double skip_start, skip_start_live, skip_step, skip_step_live, skip_mb;   // mma_kernel, SKIP form: + the share of live waves
+    double wide_start, wide_step, wide_mb;                                    // mma_kernel: MB past 34
+};
+constexpr Mma256Time TIME_256 = {17, 1.65, 0.21, 11.5, 6, 0.5, 1.25, 0.33, 27, 1.6, 0.7};
+constexpr Mma256Time TIME_256_F16 = {14, 1.6, 0.21, 9.8, 4.5, 0.7, 1.05, 0.35, 27, 1.65, 0.8};
+constexpr Mma256Time TIME_256_EX = {21.5, 2.33, 0.16, 0, 0, 0, 0, 0, 30.5, 2.85, 0.7};   // (never in the SKIP form)
+
+bool mma_wide256(const pa_hip_shape * s, const uint32_t * nkeys, int n_pages) {
+    if (s->hd != 256 || s->rows <= 64) return false;
+    const MmaForm f = mma_form(s, false), w = mma_form(s, true);
+    uint64_t tiles = 0;
+    for (int i = 0; i < n_pages; i++) tiles += (nkeys[i] + 31ull) / 32;
+    if (f.ex ? s->rows <= 512 || tiles < 384 : std::max(512u, s->rows) * tiles < 512u * 384u) return false;
+    const Mma256Time & c = f.ex ? TIME_256_EX : s->fmt == PA_FMT_F16 ? TIME_256_F16 : TIME_256;
+    auto steps = [&](const MmaForm & g, uint64_t t, uint64_t & n) {
+        const uint64_t resident = 2048u / g.nw, want = std::min(std::max<uint64_t>(1, resident / g.units), mma_chunks(g, t));
+        const uint64_t tpc = (t + want - 1) / want;
+        n = (t + tpc - 1) / tpc;
+        return (double) ((n * g.units + resident - 1) / resident * tpc);
+    };
+    double narrow = 0, wide = 0;
+    for_launches(nkeys, n_pages, [&](int, int, uint64_t t, uint64_t) {
+        uint64_t n;
+        double st = steps(f, t, n);
+        if (n * f.units <= 256) st /= TWO_PER_CU;
+        narrow += c.start + c.step * st + (n > 1 ? c.mb * f.slot_mb * n : 0) + (n > 64 ? 3.3 : 0);
+        st = steps(w, t, n);
+        if (s->rows <= 224) {
+            const double live = (double) ((s->rows + 31) / 32) / 8;
+            wide += c.skip_start + c.skip_start_live * live + (c.skip_step + c.skip_step_live * live) * st + c.skip_mb * w.slot_mb * n +
+                    (n > 64 ? 3.3 : 0);
+        } else {
+            wide += c.wide_start + c.wide_step * st + c.wide_mb * std::max(0.0, w.slot_mb * n - 34) + (n > 64 ? 2.1 : 0);
+        }
+    });
+    return wide < narrow;
+}
+
 // the matrix-core kernels, over chunks of 32-key tiles: mma_kernel (row blocks of 32*NW rows) for every head-dim-128 call
 // that attn_decode does not take and for long head-dim-256 contexts above 64 rows; mma256_kernel (row blocks of 64 rows) for
 // the other head-dim-256 calls
 int attn_mma(Call & cx, const pa_hip_shape * s, const void * const * k_pages, const void * const * v_pages,
              const uint32_t * nkeys, int n_pages, const float * Q, float * O, float * m, float * l, hipStream_t st) {
-    // mma_kernel: 32 rows per wave, 8 waves above 128 rows (prefill) and at head dim 256, 4 otherwise (verify, short verify
-    // blocks, f16 decode). mma256_kernel: 16 rows per wave, 4 waves (the reference's 48 rows per KV head fill three).
-    // Head dim 256 above 64 rows: each 16-row wave reads a whole tile from LDS for half the rows and each 64-row block
-    // dequantizes it again, but an 8-wave workgroup starts and ends 8-10 us later, so mma_kernel is taken for long contexts,
-    // the more rows the sooner. us per call, mma256_kernel against mma_kernel, fp16 operands: 16,384 q8_0 keys, 72 rows 33.0 /
-    // 26.5, 300 rows 58.1 / 56.3, 512 rows 76.7 / 77.4, 900 rows 129.7 / 99.3; 4,096 keys, 72 rows 21.1 / 22.2, 300 rows 34.9
-    // / 40.8, 900 rows 49.0 / 49.4; 1,000 keys, 300 rows 20.8 / 32.1. Exact block dots (ggml's rounding over quantized K),
-    // whose 32-row form converts and scales each dot in vector instructions: 16,384 keys, 192 rows 54.0 / 64.4, 512 rows 99.3 /
-    // 100.1, 600 rows 128.5 / 115.6, 900 rows 174 / 135; 4,096 keys, 900 rows 61 / 68.
-    uint64_t call_tiles = 0;
-    for (int i = 0; i < n_pages; i++) call_tiles += (nkeys[i] + 31ull) / 32;
-    const bool ex = s->qmode == PA_QMODE_GGML && s->fmt != PA_FMT_F16;
-    const bool wide = s->rows > 64 && (ex ? s->rows > 512 && call_tiles >= 384 : std::max(512u, s->rows) * call_tiles >= 512u * 384u);
-    const bool h256 = s->hd == 256 && !wide;
-    const uint32_t nw = h256 ? 4u : s->rows > 128 || s->hd == 256 ? 8u : 4u, rpw = h256 ? 16u : 32u;
-    const uint32_t nrb = (s->rows + rpw * nw - 1) / (rpw * nw);
+    const MmaForm form = mma_form(s, mma_wide256(s, nkeys, n_pages));
+    const uint32_t nw = form.nw, rpw = form.rpw, nrb = form.nrb, units = form.units;
+    const bool h256 = form.h256;
     // rows per KV head in the slots: whole row blocks, at head dim 256 multiples of 64 under either kernel (only real rows
     // are written)
     const uint32_t qr = s->hd == 256 ? (s->rows + 63) / 64 * 64 : nrb * rpw * nw;
     // one row block with waves past the last row: those waves only stage (with several row blocks the full ones set
     // the time, and the staging-only branch would slow them)
     const bool skip = nrb == 1 && s->rows <= rpw * (nw - 1);
-    const uint32_t units = s->nkv * nrb;
     const uint64_t rows_per_slot = (uint64_t) s->nkv * qr;
-    // key chunks: by default one round of resident workgroups (one of 8 waves or two of 4 per CU, 256 CUs); a second,
-    // partial round costs more than the extra slots save
-    const uint64_t target = cx.mma_workgroups > 0 ? (uint64_t) cx.mma_workgroups : 256u * 8 / nw;
-    // Fewer chunks where a short context does not pay for them. One chunk, written directly, takes every tile in turn and saves
-    // the slots and the merge: us with one / several, 8 heads x 129 rows in exact block dots over 64 q8_0 keys 11.9 / 13.1, over
-    // 128 keys 14.4 / 13.8; 2,000 rows over 320 keys 24.1 / 27.2. n chunks take tiles / n steps, and their slots are written
-    // and read again, so the cost is least at n = the root of tiles x slot time / step. Of the 4-wave workgroups a round holds
-    // two per CU: between one and two, the CUs that hold two set the time while the chunks are longer than a whole round's, so
-    // it is one at most, or the round: us with 64 / 43 / 32 chunks, 8 heads x 96 rows over 8,192 q8_0 keys 24.0 / 25.4 / 21.9;
-    // with 32 / 22 / 16, head dim 256, 4 heads x 256 rows over 4,096 keys 32.2 / 33.5 / 26.7.
-    auto pays = [&](uint64_t tiles) -> uint64_t {
-        const MmaTile & tile = s->hd == 128 ? (nw == 4 ? (ex ? TILE_128_W4_EX : TILE_128_W4) : ex ? TILE_128_W8_EX : TILE_128_W8)
-                             : h256 ? (ex ? TILE_256_EX : TILE_256) : ex ? TILE_256_WIDE_EX : TILE_256_WIDE;
-        const double slot_mb = (double) s->nkv * s->rows * (s->hd * sizeof(float) + sizeof(float2)) * 1e-6;
-        if (tiles * tile.only <= MERGE_US + MERGE_US_PER_MB * slot_mb) return 1;
-        const double slot_us = SLOT_US_PER_MB * slot_mb;
-        // tiles per chunk: the better of the two counts around the root, at most one workgroup per CU
-        const uint64_t round = std::max<uint64_t>(1, target / units), single = std::max<uint64_t>(1, 256 / units);
-        auto cost = [&](uint64_t t, double step) { return t * step + (tiles + t - 1) / t * slot_us; };
-        uint64_t t = std::max<uint64_t>(1, (uint64_t) std::sqrt(tiles * slot_us / tile.step));
-        if (cost(t + 1, tile.step) < cost(t, tile.step)) t++;
-        t = std::max(t, (tiles + single - 1) / single);
-        if (nw == 4) {
-            const uint64_t tr = (tiles + round - 1) / round;
-            const double step = (tiles + tr - 1) / tr * units > 256 ? TWO_PER_CU * tile.step : tile.step;
-            if (cost(tr, step) < cost(t, tile.step) + tile.gain) return round;
-        }
-        return (tiles + t - 1) / t;
-    };
+    const uint64_t target = cx.mma_workgroups > 0 ? (uint64_t) cx.mma_workgroups : 2048u / nw;
     auto chunking = [&](uint64_t tiles, uint64_t cap, uint32_t & tpc) {
         uint64_t want = std::max<uint64_t>(1, std::min(target / units, cap));
-        if (cx.mma_workgroups == 0) want = std::min(want, pays(tiles));
+        if (cx.mma_workgroups == 0) want = std::min(want, mma_chunks(form, tiles));
         tpc = (uint32_t) ((tiles + want - 1) / want);
         if (cx.chunk_keys > 0 && cx.mma_workgroups == 0)             // keys per chunk asked for, within the slot cap
             tpc = (uint32_t) std::max<uint64_t>((tiles + std::min(cap, tiles) - 1) / std::min(cap, tiles),
