@@ -40,7 +40,8 @@ namespace pa_hip {
 
 // LDS geometry per head dim: K row stride 2 HD + 16 B (EX: the raw quants, HD + 16 B), so that 16 consecutive keys' 16-byte
 // reads hit distinct banks; V row stride 2 HD + 64 B, so that the 4 rows x 64 bytes of a half-wave's transposing reads do;
-// and for EX the tile's K block scales [key][HD / 32 blocks] fp16. A stage holds 19,200 B at head dim 128, 35,840 at 256.
+// and for EX the tile's K block scales, at head dim 128 [key][4 blocks] fp16, at 256 [8 blocks][key] fp32. A stage holds 19,200 B
+// at head dim 128, 36,352 at 256.
 template <int HD> struct MmGeom {
     static constexpr int NBLK = HD / 32;                      // quant blocks per head row
     static constexpr int KST = 2 * HD + 16, KST8 = HD + 16, VST = 2 * HD + 64;
@@ -203,7 +204,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     const bool wlive = !SKIP || rb * (32 * RW) + 32 * rw < a.rows;    // uniform: the wave has a live row
 
     // ---- staging units of this thread: u = tid + NT*i -> tensor u / (64 NBLK) (uniform),
-    // key u / (2 NBLK) & 31, block (u >> 1) & (NBLK - 1), half u & 1; rows past the page's end reload its last row (masked later)
+    // key u / (2 NBLK) & 31, block (u >> 1) & (NBLK - 1), half u & 1; rows past the page's end read zeros (masked later)
     using F = MmFmt<FMT>;
     // the tensor of unit i. With one unit per thread waves 0-3 stage V and waves 4-7 K: V costs the dequantization, and the
     // SIMDs' issue favours the older of its two waves (w and w + 4), so the older one takes it
@@ -308,7 +309,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     for (int b = 0; b < NBLK; b++) dqb[b] = dcb[b] = 0u;
     if constexpr (EX) mm_prep_qi8<HD, FMT>(a, h, row, rlive, h2, Qi, dqb, dcb);
     else mm_prep_q<HD>(a, h, row, rlive, h2, Qf);
-    // EX: the B operands of the scale products. All four products share one A operand, key n's block scales at k = 2b and
+    // EX at head dim 128: the B operands of the scale products. All four products share one A operand, key n's block scales at k = 2b and
     // 2b + 1 (lanes h2 = b / 2, register b % 2), so block b's B operand holds row n's (hi, lo) pair there, zero elsewhere
     // (one operand per block in otherwise zero registers took four permutes, four selects and eleven moves per tile more)
     pa_u2 dqw[4];
@@ -593,10 +594,12 @@ static hipError_t launch_mma_128(int fmt, int nw, bool skip, int streams, const 
     return hipErrorInvalidValue;
 }
 
+// (the exact block dots at head dim 256 are taken above 512 rows only: every wave of one of their row blocks at least has rows)
 template <int FMT, bool EX>
 static hipError_t launch_mma_256_fmt(bool skip, const AttnArgs & a, uint32_t grid, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
-    if (skip) hipExtLaunchKernelGGL((mma_kernel<256, FMT, 8, true, EX>), dim3(grid), dim3(512), 0, st, ev0, ev1, 0, a);
-    else hipExtLaunchKernelGGL((mma_kernel<256, FMT, 8, false, EX>), dim3(grid), dim3(512), 0, st, ev0, ev1, 0, a);
+    if (!skip) hipExtLaunchKernelGGL((mma_kernel<256, FMT, 8, false, EX>), dim3(grid), dim3(512), 0, st, ev0, ev1, 0, a);
+    else if constexpr (!EX) hipExtLaunchKernelGGL((mma_kernel<256, FMT, 8, true, EX>), dim3(grid), dim3(512), 0, st, ev0, ev1, 0, a);
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
