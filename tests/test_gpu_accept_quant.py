@@ -73,8 +73,8 @@ def test_accept_edge_values(ws):
 
 @pytest.mark.parametrize("vocab", [1, 3, 4, 255, 1024, 16383, 16384, 16385, 16388, 50001, 50004])
 def test_accept_segment_edges(ws, vocab):
-    """Both load widths around whole segments (16,384 values): the largest value, ties, -0 == +0, NaN of either sign and
-    rows of -inf at the first and last places of a segment, against numpy.argmax."""
+    """Both load widths, 6 to 36 rows of every segment size (the largest, 16,384, from 50,001 values on): the largest value,
+    ties, -0 == +0, NaN of either sign and rows of -inf at the first, middle and last places of a row, against numpy.argmax."""
     rng = np.random.default_rng(vocab)
     at = sorted({0, 1 % vocab, vocab // 2, max(0, vocab - 2), vocab - 1, min(16383, vocab - 1), min(16384, vocab - 1)})
     rows = [np.full(vocab, -np.inf, np.float32)]
@@ -91,14 +91,48 @@ def test_accept_segment_edges(ws, vocab):
     assert np.array_equal(am, np.argmax(logits, axis=1))
 
 
-def test_accept_several_segments_per_workgroup(ws):
-    """64 rows of 13 segments: 832 workgroups of one segment become 256 of four, the last one shorter."""
-    vocab, n = 12 * 16384 + 5, 64
+def segment(n_rows, vocab):
+    """The host's segment size: the smallest that keeps to 140 workgroups, else the largest."""
+    for seg in (4096, 8192):
+        if n_rows * -(-vocab // seg) <= 140:
+            return seg
+    return 16384
+
+
+@pytest.mark.parametrize("seg,n,vocab", [(s, n, m * s + d) for s, n, m in ((4096, 5, 3), (8192, 20, 4), (16384, 33, 3))
+                                         for d in (-4, -1, 0, 1, 4)])
+def test_accept_around_each_segment(ws, seg, n, vocab):
+    """Each segment size in both load widths, rows that end just before, at and just past a segment: every row's largest value, a
+    tie behind it or its first NaN at the last place of one segment and the first of the next."""
+    assert segment(n, vocab) == seg
+    rng = np.random.default_rng(vocab)
+    logits = rng.standard_normal((n, vocab)).astype(np.float32)
+    at = [p for p in (0, 3, 4, seg - 1, seg, seg + 1, 2 * seg - 1, 2 * seg, vocab - 2, vocab - 1)]
+    for i in range(n):
+        p, kind = at[i % len(at)], i % 3
+        logits[i, p] = np.nan if kind == 2 else 50.0
+        if kind == 1:
+            logits[i, at[(i + 3) % len(at)]] = 50.0
+        if kind == 2:
+            logits[i, at[(i + 5) % len(at)]] = -np.nan
+    print(f"accept seg={seg} rows={n} vocab={vocab}", flush=True)
+    am = gpu_accept(ws, logits, np.zeros(n - 1, np.int32))[2]
+    assert np.array_equal(am, np.argmax(logits, axis=1))
+
+
+@pytest.mark.parametrize("vocab", [12 * 16384 + 5, 12 * 16384 + 4, 262144])
+def test_accept_several_segments_per_workgroup(ws, vocab):
+    """64 rows of 13 or 16 segments: 832 or 1,024 workgroups of one segment become 256 of four (the last one shorter), in both
+    load widths; ties and NaN in different segments of one workgroup and across workgroups."""
+    n = 64
     rng = np.random.default_rng(77)
     logits = rng.standard_normal((n, vocab)).astype(np.float32)
     at = rng.integers(0, vocab, n); at[:4] = [0, vocab - 1, 4 * 16384 - 1, 4 * 16384]
     logits[np.arange(n), at] = 50.0
     logits[5, at[5]:] = np.nan
+    for i, (p, q) in enumerate([(16383, 16384), (100, 3 * 16384 + 7), (2 * 16384, 4 * 16384), (16384 + 5, vocab - 1)]):
+        logits[8 + 2 * i, [p, q]] = 60.0                               # a tie: the lower index
+        logits[9 + 2 * i, q] = np.nan; logits[9 + 2 * i, p] = -np.nan   # the first NaN
     am = gpu_accept(ws, logits, np.zeros(n - 1, np.int32))[2]
     assert np.array_equal(am, np.argmax(logits, axis=1))
 

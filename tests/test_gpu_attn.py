@@ -85,10 +85,10 @@ def test_mma256_row_blocks(ws, fmt, rows):
 @pytest.mark.parametrize("fmt,rows,qmode", [(f, r, bb.QMODE_F16) for f in (bb.FMT_Q8_0, bb.FMT_Q4_0, bb.FMT_F16) for r in (65, 224, 225, 257)]
                          + [(f, r, bb.QMODE_GGML) for f in (bb.FMT_Q8_0, bb.FMT_Q4_0) for r in (513, 577)])
 def test_head256_wide_rows(ws, fmt, rows, qmode):
-    """Head dim 256 in 32-row waves (256-row blocks; above 64 rows, with the exact block dots above 512, from 384 tiles on):
-    the first rows past the 64-row blocks, the last count with idle waves, the first without, a second or third row block of
-    one row or wave; over pages that end inside a tile, hold less than one or nothing, in the default chunks, in one chunk
-    per row block (every page change inside the workgroup) and in chunks of one or two tiles."""
+    """Head dim 256 above 64 rows over one head and 387 tiles, about where the host weighs 64-row blocks against 256-row ones:
+    the first rows past a 64-row block, the last count with idle waves, the first without, a further row block of one row or
+    wave; over pages that end inside a tile, hold less than one or nothing, in the default chunks, in one chunk per row block
+    (every page change inside the workgroup) and in chunks of one or two tiles."""
     page_keys = [500, 7, 0, 64, 11740]
     nk, nkv = sum(page_keys), 1
     print(f"case fmt={fmt} rows={rows} qmode={qmode} nk={nk}", flush=True)
@@ -104,6 +104,63 @@ def test_head256_wide_rows(ws, fmt, rows, qmode):
             ws.set_split()
         eo, em, el = orc.rel_err(O, m, l, *ref)
         assert eo < TOL and em < TOL and el < TOL, (workgroups, eo, em, el)
+
+
+def run_and_check_rows(ws, fmt, nkv, rows, hd, page_keys, pick, seed, qmode, rs_pad=0, outliers=0, workgroups=(0,)):
+    """A call of many rows over a long context, checked at the rows `pick` of every head (the oracle runs those only): each
+    row's result depends on its own query."""
+    nk = sum(page_keys)
+    print(f"case fmt={fmt} nkv={nkv} rows={rows} hd={hd} nk={nk} qmode={qmode} pages={len(page_keys)}", flush=True)
+    K, V, Q, rs = case(fmt, nkv, rows, hd, nk, seed, rs_pad, 1.0, outliers)
+    shape = bb.make_shape(nkv, rows, hd, fmt, qmode, rs=rs)
+    at = np.concatenate([h * rows + np.asarray(pick) for h in range(nkv)])
+    oshape = orc.make_shape(nkv, len(pick), hd, fmt, orc.QMODE_F16 if qmode == bb.QMODE_F16 else orc.QMODE_GGML, rs=rs)
+    ref = (orc.attn_exact if qmode == bb.QMODE_F16 else orc.attn_ggml)(oshape, np.ascontiguousarray(Q[at]), K, V, nk)
+    pages = bb.pages_from_rows(K, V, rs, page_keys)
+    n = nkv * rows
+    dq, do, dml = bb.DeviceBuffer.from_array(Q), bb.DeviceBuffer(n * hd * 4), bb.DeviceBuffer(n * 8)
+    try:
+        for w in workgroups:
+            ws.set_split(mma_workgroups=w)
+            do.upload(np.full(n * hd * 4, 0x7f, np.uint8))
+            ws.attn(shape, pages, dq.ptr, do.ptr, dml.ptr, dml.ptr + n * 4)
+            bb.device_sync()
+            O, ml = do.download(np.float32).reshape(n, hd), dml.download(np.float32)
+            eo, em, el = orc.rel_err(O[at], ml[:n][at], ml[n:][at], *ref)
+            assert eo < TOL and em < TOL and el < TOL, (w, eo, em, el)
+    finally:
+        ws.set_split()
+        pages.close()
+
+
+# head dim 256 where 256-row blocks (mma_kernel) are clearly the faster ones, so that the host's estimate takes them: 65-128
+# rows over 4 heads from 16,000 keys, 200 rows from 32,000, more rows and heads over 16,000-33,000; in exact block dots above 512
+WIDE = [(bb.FMT_Q8_0, bb.QMODE_F16, 4, 65, 16100), (bb.FMT_Q4_0, bb.QMODE_F16, 3, 96, 24100), (bb.FMT_F16, bb.QMODE_F16, 4, 97, 24100),
+        (bb.FMT_F16, bb.QMODE_GGML, 4, 72, 24100), (bb.FMT_Q8_0, bb.QMODE_F16, 4, 200, 33100), (bb.FMT_Q4_0, bb.QMODE_F16, 4, 224, 33100),
+        (bb.FMT_F16, bb.QMODE_GGML, 4, 257, 33100), (bb.FMT_Q4_0, bb.QMODE_F16, 4, 225, 33100), (bb.FMT_Q8_0, bb.QMODE_F16, 3, 513, 24100),
+        (bb.FMT_F16, bb.QMODE_F16, 2, 1100, 24100), (bb.FMT_Q8_0, bb.QMODE_GGML, 2, 769, 33100), (bb.FMT_Q4_0, bb.QMODE_GGML, 3, 545, 33100)]
+
+
+@pytest.mark.parametrize("fmt,qmode,nkv,rows,nk", WIDE)
+def test_head256_long_contexts(ws, fmt, qmode, nkv, rows, nk):
+    """256-row blocks at head dim 256: several KV heads (their place in the pages, Q, the slots and the result), padded rows,
+    outlier keys in the exact block dots, f16 K in ggml's rounding (the scale multiplies the score), idle waves or none, a
+    last row block of one row or wave, pages that end inside a tile or hold nothing; in the default chunks and in one per row
+    block."""
+    exact = qmode == bb.QMODE_GGML and fmt != bb.FMT_F16
+    pages = [4096, 500, 7, 0, 64, 4096, 1000]
+    pages += [nk - sum(pages)]
+    edge = {0, 1, 31, 32, 63, 64, rows // 2, rows - 2, rows - 1} | {r for r in (255, 256, 511, 512) if r < rows}
+    run_and_check_rows(ws, fmt, nkv, rows, 256, pages, sorted(edge), 2600 + rows + fmt, qmode, rs_pad=48, outliers=4 if exact else 0,
+                       workgroups=(0, 1))
+
+
+@pytest.mark.parametrize("fmt,qmode,rows", [(bb.FMT_Q8_0, bb.QMODE_F16, 72), (bb.FMT_Q4_0, bb.QMODE_GGML, 1100)])
+def test_head256_over_two_launches(ws, fmt, qmode, rows):
+    """256-row blocks over 150 pages: two launches into one slot array."""
+    r = np.random.default_rng(rows)
+    pages = [int(x) for x in r.integers(200, 330, size=150)]
+    run_and_check_rows(ws, fmt, 4, rows, 256, pages, [0, 33, 64, rows - 1], 2800 + rows, qmode)
 
 
 @pytest.mark.parametrize("nkv,rows,hd,nk", [(8, 128, 128, 1000), (8, 1000, 128, 2049), (4, 48, 256, 4096), (4, 300, 256, 70), (8, 64, 128, 33)])

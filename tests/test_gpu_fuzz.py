@@ -5,6 +5,9 @@ prefill row blocks), head dim, format, query rounding, row padding, ragged pages
 one launch's worth of pages) and, for some, a forced split-K geometry (ws.set_split). Sizes keep the oracle within
 about a second per case.
 
+Further draws of long contexts (the oracle runs a few rows of each): head dim 256 with 65-1,200 rows, where the host weighs
+64-row against 256-row blocks, and head dim 128 with up to 64 rows, whose workgroups take two tile streams.
+
 Tolerance 2e-3 as everywhere, on inputs inside the regimes the fixed tests pin at that bar: x8 outlier channels only
 where the scores are exact block dots (q8_0 / q4_0 in ggml rounding: every kernel, every row count and head dim)."""
 import numpy as np
@@ -12,10 +15,11 @@ import pytest
 
 import backburner_amd as bb
 import oracle as orc
-from tests.test_gpu_attn import run_and_check
+from tests.test_gpu_attn import run_and_check, run_and_check_rows
 
 pytestmark = pytest.mark.gpu
 N_CASES = 48
+N_LONG = 16
 
 
 def draw(i: int):
@@ -70,9 +74,40 @@ def test_random_geometry(ws, i):
     print(f"fuzz case {i}: max rel err O {eo:.3e} m {em:.3e} l {el:.3e}", flush=True)
 
 
+def draw_long(i: int):
+    """Long contexts, by turns at head dim 256 above 64 rows and at head dim 128 up to 64 rows."""
+    r = np.random.default_rng(5000 + i)
+    fmt = int(r.choice([bb.FMT_Q8_0, bb.FMT_Q4_0, bb.FMT_F16]))
+    qmode = int(r.choice([bb.QMODE_GGML, bb.QMODE_F16]))
+    if i % 2 == 0:
+        hd, nkv, nk = 256, int(r.choice([2, 3, 4])), int(r.integers(20000, 34000))
+        rows = int(r.integers(65, 129)) if i % 4 == 0 else int(r.integers(600, 1200))
+        if rows <= 512 and qmode == bb.QMODE_GGML:
+            fmt = bb.FMT_F16                                         # (the exact block dots go there above 512 rows)
+    else:
+        hd, nkv, nk, rows = 128, int(r.choice([1, 3, 8])), int(r.integers(12000, 30000)), int(r.integers(9, 65))
+    cuts = np.sort(r.integers(0, nk, size=int(r.integers(3, 9))))
+    pages = [int(x) for x in np.diff(np.concatenate([[0], cuts, [nk]]))]
+    exact = fmt != bb.FMT_F16 and qmode == bb.QMODE_GGML
+    # the default split, and for two tile streams (from 10 tiles per chunk, 32 up to 32 rows) one of a few chunks per head
+    splits = (0,) if hd == 256 else (0, nkv * int(r.integers(1, 9)))
+    return dict(fmt=fmt, hd=hd, qmode=qmode, nkv=nkv, rows=rows, pages=pages, rs_pad=int(r.choice([0, 16, 48])),
+                outliers=4 if exact else 0, splits=splits)
+
+
+@pytest.mark.parametrize("i", range(N_LONG))
+def test_random_long_context(ws, i):
+    c = draw_long(i)
+    print(f"fuzz long case {i}: {c}", flush=True)
+    pick = sorted({0, 31, 33, c["rows"] // 2, c["rows"] - 1} & set(range(c["rows"])))
+    run_and_check_rows(ws, c["fmt"], c["nkv"], c["rows"], c["hd"], c["pages"], pick, 9000 + i, c["qmode"], rs_pad=c["rs_pad"],
+                       outliers=c["outliers"], workgroups=c["splits"])
+
+
 def test_draws_cover_the_kernels():
     """The draws reach every routing branch: the decode kernel (even heads, <= 8 rows, ggml rounding, hd 128), the
-    4- and 8-wave matrix-core kernels, the head-dim-256 kernels in both roundings, more than 128 pages (two launches), forced splits."""
+    4- and 8-wave matrix-core kernels, the head-dim-256 kernels in both roundings, more than 128 pages (two launches), forced
+    splits; the long ones 256-row blocks at head dim 256 (in both roundings, with and without idle waves) and two tile streams."""
     cs = [draw(i) for i in range(N_CASES)]
     dec = [c for c in cs if c["hd"] == 128 and c["rows"] <= 8 and c["nkv"] % 2 == 0 and c["fmt"] != bb.FMT_F16
            and c["qmode"] == bb.QMODE_GGML]
@@ -85,3 +120,12 @@ def test_draws_cover_the_kernels():
     assert any(c["nkv"] >= 16 for c in dec) and any(c["nkv"] >= 16 and c not in dec for c in cs)
     assert any(c["split"] for c in cs) and any(c["outliers"] for c in cs)
     assert any(c["outliers"] and c["rows"] > 128 for c in cs) and any(c["outliers"] and c["hd"] == 256 for c in cs)
+    long = [draw_long(i) for i in range(N_LONG)]
+    wide = [c for c in long if c["hd"] == 256 and sum(c["pages"]) >= 512 * 32]
+    assert any(c["rows"] <= 224 for c in wide) and any(c["rows"] > 512 for c in wide)
+    assert any(c["rows"] > 512 and c["fmt"] != bb.FMT_F16 and c["qmode"] == bb.QMODE_GGML for c in wide)
+    assert any(c["fmt"] == bb.FMT_F16 and c["qmode"] == bb.QMODE_GGML for c in wide) and any(c["qmode"] == bb.QMODE_F16 for c in wide)
+    two = [c for c in long if c["hd"] == 128 and sum(c["pages"]) / 32 / (c["splits"][1] / c["nkv"]) > 33]
+    assert any(c["rows"] <= 32 for c in two) and any(c["rows"] > 32 for c in two)
+    assert any(c["qmode"] == bb.QMODE_F16 or c["fmt"] == bb.FMT_F16 for c in two)
+    assert any(c["qmode"] == bb.QMODE_GGML and c["fmt"] != bb.FMT_F16 for c in two)

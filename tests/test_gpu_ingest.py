@@ -149,6 +149,36 @@ def test_append_over_many_pages(nkv, hd, fmt):
             pages.close()
 
 
+@pytest.mark.parametrize("page", [40000, 4096])
+@pytest.mark.parametrize("store_f16", [False, True])
+def test_append_of_more_rows_than_a_grid_holds(page, store_f16):
+    """70,001 rows: past 65,535 rows (a grid dimension) in pages of 40,000 keys, past 16 pages (a launch's) in pages of 4,096."""
+    nkv, hd, pos0, n = 1, 128, 5, 70001
+    n_pages = (pos0 + n + page - 1) // page
+    fmt = bb.FMT_Q8_0 if store_f16 else bb.FMT_Q4_0
+    X = np.random.default_rng(page).standard_normal((n, nkv, hd), dtype=np.float32)
+    hb = orc.head_bytes(fmt, hd); rs = nkv * hb
+    out_rs = nkv * hd * 2 if store_f16 else rs
+    print(f"append {n} rows page={page} store_f16={store_f16}", flush=True)
+    rows = orc.rows_from_f32(fmt, X, rs, hb)
+    pages = bb.alloc_pages(n_pages, page * out_rs)
+    try:
+        shape = bb.make_shape(nkv, 8, hd, fmt, rs=rs)
+        if store_f16:
+            dR = bb.DeviceBuffer.from_array(rows)
+            bb.append_rows(shape, pages, page, pos0, dR.ptr, dR.ptr, n, store_f16=True)
+            want = orc.store_rows_f16(rows, n, nkv, hd, rs, hb).view(np.uint8).reshape(-1)
+        else:
+            dX = bb.DeviceBuffer.from_array(X)
+            bb.append_f32(shape, pages, page, pos0, dX.ptr, dX.ptr, n)
+            want = rows
+        bb.device_sync()
+        for got in page_bytes(pages, n_pages, page * out_rs):
+            assert np.array_equal(got[pos0 * out_rs:(pos0 + n) * out_rs], want)
+    finally:
+        pages.close()
+
+
 def test_append_rejects_positions_past_the_pages():
     shape = bb.make_shape(8, 8, 128, bb.FMT_Q8_0)
     pages = bb.alloc_pages(1, PAGE_KEYS * shape.rs)
