@@ -199,13 +199,17 @@ namespace {
 constexpr int DEC_TARGET_WG_Q8 = 768, DEC_TARGET_WG_Q4 = 1024;
 
 // The split of the matrix-core kernels (mma_chunks): what a step of one tile costs with one workgroup on a CU (TWO_PER_CU times it
-// with two), what a tile of a call's only chunk costs, the gain below which 4-wave calls keep the larger count, and the longest
-// chunk, in tiles, with which they take one workgroup per CU; the slots' time, written and read back; and what a merge costs,
-// with its share per MB of result. Fitted to 3,600 shapes of 12 to 4,000 rows, 1 to 32 heads and 64 to 33,333 keys.
-struct MmaTile { double step, only, gain; uint32_t alone; };
-constexpr MmaTile TILE_128_W4 = {0.8, 1.25, 0, 10}, TILE_128_W4_EX = {1.1, 1.7, 0, 10}, TILE_128_W8 = {1.5, 1.4}, TILE_128_W8_EX = {1.5, 1.8};
-constexpr MmaTile TILE_256 = {1.2, 1.75, 1, 12}, TILE_256_EX = {1.7, 2.4, 1, 10}, TILE_256_WIDE = {1.4, 1.75},
-                  TILE_256_WIDE_SKIP = {2.4, 1.75}, TILE_256_WIDE_EX = {2.6, 2.4};
+// with two), what a tile of a call's only chunk costs, what a step costs more where every tile is taken against its own maximum
+// (attn_mma: chunks longer than the round's, where those are of up to OWN_REF_TILES tiles), the gain below which calls keep
+// the larger count, and for 4-wave kernels the longest chunk, in tiles, with which they take one workgroup per CU; the slots'
+// time, written and read back; and what a merge costs, with its share per MB of result. Fitted to 3,600 shapes of 12 to 4,000
+// rows, 1 to 32 heads and 64 to 33,333 keys.
+struct MmaTile { double step, only, own, gain; uint32_t alone; };
+constexpr MmaTile TILE_128_W4 = {0.8, 1.5, 0.1, 0, 10}, TILE_128_W4_EX = {1.1, 1.9, 0.1, 0, 10};
+constexpr MmaTile TILE_128_W8 = {1.5, 1.6, 0.25}, TILE_128_W8_EX = {1.5, 2.1, 0.4};
+constexpr MmaTile TILE_256 = {1.2, 2.1, 0.1, 1, 12}, TILE_256_EX = {1.7, 2.6, 0.1, 1, 6}, TILE_256_WIDE = {1.4, 2.1},
+                  TILE_256_WIDE_SKIP = {2.4, 2.1}, TILE_256_WIDE_EX = {2.6, 2.6};
+constexpr uint32_t OWN_REF_TILES = 4;
 constexpr double TWO_PER_CU = 1.3, SLOT_US_PER_MB = 0.444, MERGE_US = 4.6, MERGE_US_PER_MB = 2.8;
 
 // One call of the engine path: where its split-K slots go, its geometry overrides, its timing events and, for
@@ -403,15 +407,21 @@ uint64_t mma_chunks(const MmaForm & f, uint64_t tiles) {
     if (tiles * f.tile.only <= MERGE_US + MERGE_US_PER_MB * f.slot_mb) return 1;
     const uint64_t round = std::max<uint64_t>(1, 2048u / f.nw / f.units), single = std::max<uint64_t>(1, 256 / f.units);
     const double slot_us = SLOT_US_PER_MB * f.slot_mb;
-    const uint64_t t1 = (tiles + single - 1) / single;               // tiles per chunk with one workgroup per CU
+    const uint64_t t1 = (tiles + single - 1) / single, tr = (tiles + round - 1) / round;   // tiles per chunk, one per CU / the round
     // tiles per chunk: the better of the two counts around the root
-    auto cost = [&](uint64_t t) { return t * f.tile.step + (tiles + t - 1) / t * slot_us; };
+    const double own = tr <= OWN_REF_TILES ? f.tile.own : 0.0;
+    // (of 8 waves with 8, 16, .. chunks: a row's slots are then a power of two of bytes, and a workgroup's rows meet on the same
+    // memory channels, which costs 8 heads x 160 rows 0 or 5 us of 28, by the buffer's place)
+    auto cost = [&](uint64_t t) {
+        const uint64_t n = (tiles + t - 1) / t;
+        return t * (f.tile.step + (t > tr ? own : 0.0)) + n * slot_us + (f.nw == 8 && n >= 8 && (n & (n - 1)) == 0 ? 1.0 : 0.0);
+    };
     uint64_t t = std::max<uint64_t>(1, (uint64_t) std::sqrt(tiles * slot_us / f.tile.step));
     if (cost(t + 1) < cost(t)) t++;
     t = std::max(t, t1);
+    if (cost(t1) < cost(t) + f.tile.gain) t = t1;
     if (f.nw == 4) {
-        if (cost(t1) < cost(t) + f.tile.gain) t = t1;
-        const uint64_t tr = (tiles + round - 1) / round, n = (tiles + tr - 1) / tr;
+        const uint64_t n = (tiles + tr - 1) / tr;
         if (n * f.units > 256 && (t1 > f.tile.alone || tr * TWO_PER_CU * f.tile.step + n * slot_us < cost(t))) return n;
     }
     return (tiles + t - 1) / t;
@@ -540,6 +550,14 @@ int attn_mma(Call & cx, const pa_hip_shape * s, const void * const * k_pages, co
         a.slots = (uint32_t) n_slots;
         a.qmode = s->qmode; a.fused = direct ? 1u : 0u; a.scale = s->scale; a.s_mul = 1.4426950408889634f;
         a.q = Q; a.po = cx.po; a.pml = cx.pml; a.O = O; a.m = m; a.l = l;
+        // Fewer chunks than the round hold more tiles each, and the fp16 rounding of P costs more there: a chunk's probabilities are
+        // taken against one reference, so of its tiles' largest ones, which weigh most, only the first is exactly 1. Where the
+        // round's chunks are of few tiles, such a call takes every tile against its own maximum instead (0.1-0.3 us per tile, the
+        // rescaling of O). Error of O against 64 bits in the round / in fewer chunks / so: 8 heads x 120 rows over 983 f16 keys
+        // 1.12e-4 / 1.63e-4 / 1.12e-4, 40 rows over 1,807 q4_0 keys 1.94e-4 / 2.28e-4 / 1.94e-4; over 1,500 drawn calls fewer
+        // chunks raised it by 1-31 % on average where the round's chunks are of one tile, 0-7 % of three, 0-1 % from five on.
+        const uint64_t most = std::max<uint64_t>(1, std::min(target / units, cap)), tr = (tiles + most - 1) / most;
+        a.own_ref = cx.mma_workgroups == 0 && cx.chunk_keys == 0 && tr <= OWN_REF_TILES && tpc > tr ? 1u : 0u;
         const uint32_t grid = (a.n_items + 7) / 8 * 8;
         hipEvent_t e0 = li == 0 ? cx.ev0 : nullptr, e1 = li + 1 == n_launch ? cx.ev1 : nullptr;
         // two tile streams per workgroup (mma_kernel, NS) where half its waves have no rows and the chunk is long enough to
@@ -770,6 +788,7 @@ bool append_ok(const char * fn, const pa_hip_shape * s, void * const * kp, void 
     if (!kp || !vp) { set_err(f + ": null page table"); return false; }
     for (uint64_t pi = pos0 / page_keys; pi <= (pos0 + (uint64_t) n - 1) / page_keys; pi++)
         if (!kp[pi] || !vp[pi]) { set_err(f + ": null page " + std::to_string(pi)); return false; }
+    // (a bound of the interface: the launches split any number of rows, so no index depends on it)
     if (2ull * std::min(n, page_keys) * s->nkv * (s->hd / 32) >= (1ull << 31)) { set_err(f + ": segment too large"); return false; }
     return true;
 }

@@ -28,6 +28,7 @@ struct AttnArgs {
     uint32_t slot0;                 // slot of chunk 0 of this launch
     uint32_t slots;                 // decode / MMA kernels: the call's slot count (slots are row-major: [head, row][slot])
     uint32_t qmode;                 // PA_QMODE_GGML / PA_QMODE_F16
+    uint32_t own_ref;               // MMA kernels: 1 = every tile's probabilities against its own maximum (see attn_mma)
     uint32_t fused;                 // 1: this launch holds every chunk of the call (a single chunk writes the result)
     float scale;                    // softmax scale (PA_QMODE_F16 folds it into Q)
     float s_mul;                    // factor from the dot to base-2 logits (scale * log2 e, or log2 e)

@@ -16,6 +16,7 @@ typedef __fp16 mm_tr4 __attribute__((__vector_size__(4 * sizeof(__fp16))));
 #define MM_LDS __attribute__((address_space(3)))
 
 constexpr float MM_PMAX = 6.0f;                   // p <= 2^6 between rescales
+constexpr float MM_OWN = 20.0f;                   // own_ref: how far below the running max a tile's reference may lie
 constexpr float MM_LOG2E = 1.4426950408889634f;
 
 template <int FMT> struct MmFmt {

@@ -345,6 +345,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
     float mc = 0.0f;                                                 // EX: mref once it is finite (0 before), the shift
                                                                      // the block dots start from
     const mm_h2 one2 = {(_Float16) 1.0f, (_Float16) 1.0f};
+    const bool own = a.own_ref != 0;
+    const float pmax = own ? -INFINITY : MM_PMAX;
 
     const int q4 = lane >> 4, s4 = lane & 15;
     // a tile's K operands (A operand of S^T, lane (h2, n): key n; !EX: dims 16kk + 8h2 .. +7; EX: the quants of dims 32b +
@@ -451,9 +453,10 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void mma_kernel(const AttnArgs a) 
             tm = fmaxf(fmaxf(fmaxf(tm, t1), t2), fmaxf(fmaxf(t3, t4), S[15]));
         }
         tm = EX ? tm + mc : tm * sm;                                 // base 2
-        if (__builtin_amdgcn_ballot_w64(tm > mref + MM_PMAX)) {
-            // rare: move the reference max of every row that needs it (uniform branch)
-            float mn = fmaxf(mref, mm_max32(tm));                    // the row's other half: lane ^ 32
+        if (__builtin_amdgcn_ballot_w64(tm > mref + pmax)) {
+            // rare: move the reference max of every row that needs it (uniform branch); own_ref: to every tile's maximum
+            const float tr = mm_max32(tm);                           // the row's other half: lane ^ 32
+            float mn = own ? fmaxf(tr, mm_max32(fmaxf(mx, tm)) - MM_OWN) : fmaxf(mref, tr);
             if constexpr (EX && FMT == 2 && HD == 128) {             // a value the (hi, lo) pair of -mn holds exactly
                 const _Float16 mh = (_Float16) mn, ml = (_Float16) (mn - (float) mh);
                 mn = (float) mh + (float) ml;

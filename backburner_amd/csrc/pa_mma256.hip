@@ -4,7 +4,7 @@
 // PA_QMODE_GGML (ggml's f16 vec_dot type; the scale then multiplies the score). In PA_QMODE_GGML over quantized K
 // (EX) the scores are ggml's exact integer block dots: K staged as its integer quants with the block scales beside the
 // tile, Q as ggml's q8_0 quants times 2^-s_b; per 32-dim block one MFMA gives the integer dot and one more the
-// product of the key's and the row's block scales (see mm_prep_q in pa_mma.hip for the scale pair), summed in fp32.
+// product of the key's and the row's block scales (see mm_prep_qi8 in pa_mma.hip for the scale pair), summed in fp32.
 //
 // One workgroup = one KV head x one block of 64 query rows x one chunk of consecutive 32-key tiles; 4 waves of 16 rows
 // (48 rows: three waves compute, the fourth only stages). Per tile the workgroup dequantizes K and V once into LDS as
@@ -242,6 +242,8 @@ __global__ __launch_bounds__(256, WPS) void mma256_kernel(const AttnArgs a) {
     const float sm = a.qmode == 0 && FMT == 0 ? a.scale * MM_LOG2E : MM_LOG2E;   // score -> base-2 logit (!EX)
     float mc = 0.0f;                                                 // EX: the scores' offset, mref once finite (0 before)
     const mm_h2 one2 = {(_Float16) 1.0f, (_Float16) 1.0f};
+    const bool own = a.own_ref != 0;
+    const float pmax = own ? -INFINITY : MM_PMAX;
 
     auto compute = [&](int stage, int nvalid) {
         const char * Kt = smem + stage * M2_STAGE;
@@ -303,8 +305,9 @@ __global__ __launch_bounds__(256, WPS) void mma256_kernel(const AttnArgs a) {
         }
         float tm = fmaxf(fmaxf(fmaxf(S[0][0], S[0][1]), fmaxf(S[0][2], S[0][3])), fmaxf(fmaxf(S[1][0], S[1][1]), fmaxf(S[1][2], S[1][3])));
         tm = EX ? tm + mc : tm * sm;                                 // this lane's quarter of row n's tile max, base 2
-        if (__builtin_amdgcn_ballot_w64(tm > mref + MM_PMAX)) {
-            const float mn = fmaxf(mref, mm_max32(m2_max16(tm)));    // the row's other keys: lanes n + 16 i
+        if (__builtin_amdgcn_ballot_w64(tm > mref + pmax)) {         // (own_ref: to every tile's maximum)
+            const float tr = mm_max32(m2_max16(tm));                 // the row's other keys: lanes n + 16 i
+            const float mn = own ? fmaxf(tr, mm_max32(m2_max16(fmaxf(mx, tm))) - MM_OWN) : fmaxf(mref, tr);
             const float alpha = mref == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mref - mn);
             #pragma unroll
             for (int db = 0; db < HD / 16; db++) O[db] *= alpha;

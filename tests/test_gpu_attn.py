@@ -182,6 +182,69 @@ def test_short_context_split(ws, nkv, rows, hd, nk):
         assert eo < 1e-3 and em < 1e-6 and el < 1e-3, (eo, em, el)
 
 
+@pytest.mark.parametrize("fmt,qmode,nkv,rows,hd,nk", [
+    (bb.FMT_F16, bb.QMODE_GGML, 8, 120, 128, 983), (bb.FMT_F16, bb.QMODE_F16, 8, 64, 128, 702), (bb.FMT_F16, bb.QMODE_GGML, 8, 784, 128, 256),
+    (bb.FMT_Q4_0, bb.QMODE_GGML, 8, 40, 128, 1807), (bb.FMT_Q8_0, bb.QMODE_F16, 8, 232, 128, 256), (bb.FMT_Q8_0, bb.QMODE_GGML, 4, 426, 256, 256),
+    (bb.FMT_F16, bb.QMODE_F16, 4, 48, 256, 3141), (bb.FMT_F16, bb.QMODE_F16, 4, 1236, 256, 256)])
+def test_short_context_error(ws, fmt, qmode, nkv, rows, hd, nk):
+    """A short context in fewer chunks than it has tiles is as exact as with one tile per chunk: every tile's probabilities are
+    taken against its own maximum, so that the largest of each tile is 1 in fp16 either way. The chunks then differ by fp32
+    merging only, 1e-7 of errors of 1e-4: 1 % of them is far above that (with one reference per chunk: 1.1 to 1.6 times)."""
+    print(f"case fmt={fmt} qmode={qmode} nkv={nkv} rows={rows} hd={hd} nk={nk}", flush=True)
+    K, V, Q, rs = case(fmt, nkv, rows, hd, nk, 2400 + rows, outliers=4)
+    shape = bb.make_shape(nkv, rows, hd, fmt, qmode, rs=rs)
+    ref = orc.attn_exact(orc.make_shape(nkv, rows, hd, fmt, orc.QMODE_F16 if qmode == bb.QMODE_F16 else orc.QMODE_GGML, rs=rs), Q, K, V, nk)
+    err = []
+    for workgroups in (0, 100000):                            # the default, one tile per chunk
+        ws.set_split(mma_workgroups=workgroups)
+        try:
+            O, m, l = bb.attn_host(shape, K, V, Q, ws=ws)
+        finally:
+            ws.set_split()
+        D = O.astype(np.float64) * np.exp(m.astype(np.float64) - ref[1])[:, None] - ref[0]
+        err.append(np.linalg.norm(D) / np.linalg.norm(ref[0]))
+    print(f"error of O: default {err[0]:.3e}, one tile per chunk {err[1]:.3e}", flush=True)
+    assert err[0] < 1.01 * err[1], err
+
+
+@pytest.mark.parametrize("amps", [(30, 0.01, 0.01, 0.01, 0.01, 0.01, 0.01, 0.01, 0.01, 0.01), (0.01, 0.1, 1, 3, 10, 30, 40, 50, 60, 70),
+                                  (50, 1, 50, 0.1, 20, 0.01, 60, 1, 0.01, 40), (60, 50, 40, 30, 25, 20, 15, 10, 5, 1)])
+@pytest.mark.parametrize("fmt,qmode,nkv,rows,hd", [(bb.FMT_F16, bb.QMODE_F16, 8, 1500, 128), (bb.FMT_Q8_0, bb.QMODE_GGML, 8, 1500, 128),
+                                                   (bb.FMT_Q4_0, bb.QMODE_GGML, 8, 64, 128), (bb.FMT_Q8_0, bb.QMODE_F16, 4, 1536, 256),
+                                                   (bb.FMT_Q4_0, bb.QMODE_GGML, 4, 1536, 256)])
+def test_tile_maxima_far_apart(ws, fmt, qmode, nkv, rows, hd, amps):
+    """Keys whose size changes by the tile, so that a row's tile maxima rise, fall and alternate by hundreds of powers of two
+    within one chunk: a tile's reference follows its maximum no further down than 2^20 below the row's largest, and nothing
+    overflows or is lost."""
+    nk = 32 * len(amps) - 5
+    X = np.random.default_rng(rows + hd + len(amps)).standard_normal((nk, nkv, hd), dtype=np.float32)
+    X *= np.repeat(np.array(amps, np.float32), 32)[:nk, None, None]
+    hb = orc.head_bytes(fmt, hd); rs = nkv * hb
+    K = orc.rows_from_f32(fmt, X, rs, hb)
+    V = orc.fill_rows(3, fmt, nkv, hd, nk, rs=rs)
+    Q = orc.normal(5, 0, nkv * rows * hd).reshape(nkv * rows, hd)
+    print(f"case fmt={fmt} qmode={qmode} nkv={nkv} rows={rows} hd={hd} amps={amps}", flush=True)
+    O, m, l = bb.attn_host(bb.make_shape(nkv, rows, hd, fmt, qmode, rs=rs), K, V, Q, ws=ws)
+    f16q = qmode == bb.QMODE_F16
+    ref = orc.attn_exact(orc.make_shape(nkv, rows, hd, fmt, orc.QMODE_F16 if f16q else orc.QMODE_GGML, rs=rs), Q, K, V, nk)
+    assert np.isfinite(O).all() and np.isfinite(m).all() and np.isfinite(l).all()
+    # Scores of hundreds magnify what a score is rounded by: quantized K in fp16 operands by 2^-11 of it, and the exact block dots
+    # at head dim 128, whose row scale is a pair of fp16 values, by up to |dot| dk 2^-25 per block, here 2^17 * 2 * 2^-25 = 0.8 %.
+    # Those two are compared with the same call in one tile per chunk, the others with the oracle.
+    eo, em, el = orc.rel_err(O, m, l, *ref)
+    print(f"max rel err O {eo:.2e} m {em:.2e} l {el:.2e}", flush=True)
+    if fmt == bb.FMT_F16 or (hd == 256 and not f16q):
+        assert eo < TOL and em < TOL and el < TOL, (eo, em, el)
+    else:
+        ws.set_split(mma_workgroups=100000)                   # the same scores, one tile per chunk
+        try:
+            one = bb.attn_host(bb.make_shape(nkv, rows, hd, fmt, qmode, rs=rs), K, V, Q, ws=ws)
+        finally:
+            ws.set_split()
+        eo, em, el = orc.rel_err(O, m, l, *one)
+        assert eo < 1e-3 and em < 1e-6 and el < 1e-3, (eo, em, el)
+
+
 @pytest.mark.parametrize("qmode", [bb.QMODE_GGML, bb.QMODE_F16])
 @pytest.mark.parametrize("fmt", [bb.FMT_Q8_0, bb.FMT_Q4_0, bb.FMT_F16])
 @pytest.mark.parametrize("rows", [9, 33, 64])
