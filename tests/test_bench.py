@@ -38,25 +38,27 @@ def test_committed_traffic_summary(name, kernel, alg):
     assert kernel in (ROOT / "profiles" / "bench_all_kernels.md").read_text()
 
 
-@pytest.mark.parametrize("name,kernel,flop,extra", [("prefill", "mma_kernel<1, 8, false, true>", 4 * 4096 * 65536 * 128 * 8, 1.25),
-                                                    ("prefill_f16", "mma_kernel<1, 8, false, false>", 4 * 4096 * 65536 * 128 * 8, 1.0),
-                                                    ("verify", "mma_kernel<1, 4, false, true>", 4 * 128 * 98304 * 128 * 8, 1.25),
-                                                    ("verify_q4_0", "mma_kernel<2, 4, false, true>", 4 * 128 * 143360 * 128 * 8, 1.3125),
+@pytest.mark.parametrize("name,kernel,flop,extra", [("prefill", "mma_kernel<128, 1, 8, false, true, 1>", 4 * 4096 * 65536 * 128 * 8, 1.125),
+                                                    ("prefill_f16", "mma_kernel<128, 1, 8, false, false, 1>", 4 * 4096 * 65536 * 128 * 8, 1.0),
+                                                    ("verify", "mma_kernel<128, 1, 4, false, true, 1>", 4 * 128 * 98304 * 128 * 8, 1.125),
+                                                    ("verify_q4_0", "mma_kernel<128, 2, 4, false, true, 1>", 4 * 128 * 143360 * 128 * 8, 1.1875),
                                                     ("reference_shape", "mma256_kernel<256, 1, true, false, 2>", 4 * 48 * 65536 * 256 * 4, 1.0)])
 def test_committed_mma_counters(name, kernel, flop, extra):
     """The matrix-core kernels' counter summaries: the MFMA work the counters saw (fp16 MOPS_F16 x 512 plus int8
-    MOPS_I8 x 512) is the algorithmic flops times what the form adds (the exact-dot forms one scale-product MFMA per
-    32-dim block beside the 8 QK and PV MFMAs' worth of a 32 x 32 tile, 1.25x; q4_0 one more MFMA per tile for the
-    nibble offset, 1.3125x; the exact forms take QK, half the flops, on the int8 matrix cores), K/V are fetched about
+    MOPS_I8 x 512) is the algorithmic flops times what the form adds (the exact-dot forms one scale product of 8 terms per
+    32-dim block, half an MFMA of 16, beside the 16 MFMAs' worth of QK and PV of a 32 x 32 tile, 1.125x; q4_0 one more MFMA
+    per tile for the nibble offset, 1.1875x; the exact forms take QK, half the flops, on the int8 matrix cores), K/V are fetched about
     once, and the MFMA busy fraction is derived from the raw cycle counters."""
     d = json.loads((ROOT / "profiles" / f"{name}_pmc.json").read_text())
     c = d["counters"]
     assert kernel in d["kernel"] and d["flop_per_launch"] == flop
+    assert f'pa_hip::{kernel}' in (ROOT / "bench.py").read_text()      # the kernel that bench.py reports them beside
     assert c["fp16_mfma_flops"] == c["SQ_INSTS_VALU_MFMA_MOPS_F16"] * 512
     assert c.get("int8_mfma_ops", 0) == c["SQ_INSTS_VALU_MFMA_MOPS_I8"] * 512
     work = c["fp16_mfma_flops"] + c.get("int8_mfma_ops", 0)
     assert work == pytest.approx(extra * flop, rel=1e-6)
-    if kernel.endswith("false, true>"):                                # int8 QK: exactly half the algorithmic work
+    if kernel.endswith("false, true, 1>"):                             # int8 QK: exactly half the algorithmic work
+        assert name in ("prefill", "verify", "verify_q4_0")
         assert c["int8_mfma_ops"] == flop // 2
     assert d["alg_bytes_per_launch"] <= d["traffic_bytes_per_launch"] < 1.6 * d["alg_bytes_per_launch"]
     assert 0 < c["mfma_busy_frac"] < 1 and 0 < c["MfmaUtil_pct"] < 100
